@@ -346,6 +346,32 @@ int tc_paged_rotate_keys(void* const* k_pools_host, int num_layers, const int64_
                          const float* cos_sin_host, void* stream);
 
 /* ------------------------------------------------------------------------ */
+/* Cache appends                                                             */
+/* ------------------------------------------------------------------------ */
+
+/* The append of threadcut/kv.py:68-77 in one launch: rows new tokens' K and V
+ * ([batch, heads, rows, head_dim] with element strides {batch, head, token}, a
+ * transposed view for instance) go to rows row0 .. row0 + rows of both caches
+ * [batch, heads, capacity, head_dim] (one set of strides for K and V). The
+ * rows may not overlap what is written. */
+int tc_append_rows(const void* k_rows_dev, const int64_t k_strides[3], const void* v_rows_dev,
+                   const int64_t v_strides[3], void* k_cache_dev, void* v_cache_dev,
+                   const int64_t cache_strides[3], int64_t capacity, int64_t row0, int batch,
+                   int heads, int64_t rows, int head_dim, int dtype, void* stream);
+
+/* The same into page pools, for num_layers layers in one launch (HOST arrays
+ * of device pointers; every layer's rows share one set of strides, every pool
+ * the layout of tc_decode_paged_attention). Token r of batch row b goes to
+ * slot slots_dev[b][r] = {page, slot} (int64 [batch, rows, 2] on the device,
+ * 16-byte aligned); a slot outside the pool is skipped. */
+int tc_paged_append_rows(const void* const* k_rows_host, const int64_t k_strides[3],
+                         const void* const* v_rows_host, const int64_t v_strides[3],
+                         void* const* k_pools_host, void* const* v_pools_host,
+                         const int64_t pool_strides[3], int num_pages, int page_tokens,
+                         const int64_t* slots_dev, int num_layers, int batch, int heads, int64_t rows,
+                         int head_dim, int dtype, void* stream);
+
+/* ------------------------------------------------------------------------ */
 /* Prefill attention                                                         */
 /* ------------------------------------------------------------------------ */
 

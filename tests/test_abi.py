@@ -179,6 +179,36 @@ def test_splice_validation(lib):
     assert lib.tc_shift_keys(4096, st, 8192, st, 1, 8, 0, 128, 0, table, None) == _lib.TC_OK
 
 
+def test_append_validation(lib):
+    st = _lib.i64x3(0, 1 << 20, 128)
+
+    def append(row0=0, rows=4, cap=100, k=4096, ks=st, cs=st, d=128, dt=0):
+        return lib.tc_append_rows(k, ks, 8192, st, 12288, 16384, cs, cap, row0, 1, 8, rows, d, dt, None)
+
+    assert append(row0=97) == _lib.TC_ERR_INVALID_ARGUMENT                   # past the capacity
+    assert append(row0=-1) == _lib.TC_ERR_INVALID_ARGUMENT
+    assert append(rows=-1) == _lib.TC_ERR_INVALID_ARGUMENT
+    assert append(k=0) == _lib.TC_ERR_INVALID_ARGUMENT
+    assert append(k=4100) == _lib.TC_ERR_ALIGNMENT
+    assert append(ks=_lib.i64x3(0, 1 << 20, 130)) == _lib.TC_ERR_ALIGNMENT
+    assert append(cs=_lib.i64x3(0, 1 << 20, 64)) == _lib.TC_ERR_INVALID_ARGUMENT  # cache rows would overlap
+    assert append(d=64) == _lib.TC_ERR_UNSUPPORTED
+    assert append(dt=5) == _lib.TC_ERR_UNSUPPORTED
+    assert append(rows=0, k=0) == _lib.TC_OK                                 # nothing to write
+
+    p = _lib.ptr_array([4096])
+
+    def paged(slots=4096, pages=4, P=16, k=p, layers=1):
+        return lib.tc_paged_append_rows(k, st, p, st, p, p, _lib.i64x3(8 * P * 128, P * 128, 128), pages, P, slots,
+                                        layers, 1, 8, 3, 128, 0, None)
+
+    assert paged(slots=None) == _lib.TC_ERR_INVALID_ARGUMENT
+    assert paged(slots=4104) == _lib.TC_ERR_ALIGNMENT
+    assert paged(pages=0) == _lib.TC_ERR_INVALID_ARGUMENT
+    assert paged(k=_lib.ptr_array([0])) == _lib.TC_ERR_INVALID_ARGUMENT
+    assert paged(layers=0, slots=None) == _lib.TC_OK
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "absent.so"))

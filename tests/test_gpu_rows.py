@@ -1,0 +1,113 @@
+"""The cache appends as kernels (tc_append_rows, tc_paged_append_rows) against torch's own copies: every view a
+caller may hand over lands in the same rows bit for bit, and nothing else of the buffer changes. Views that the
+kernels do not take (misaligned, another type, a broadcast batch) go through torch and give the same."""
+import pytest
+import torch
+
+from threadcut_amd import kv, paged
+
+pytestmark = pytest.mark.gpu
+
+
+def rows(form, b, h, n, dtype, dev, seed):
+    """[b, h, n, 128] new rows in one of the forms that reach an append."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    r = lambda *s: torch.randn(s, generator=g, device=dev).to(dtype)
+    if form == "heads first":
+        return r(b, h, n, 128)
+    if form == "tokens first":  # a projection's transposed view
+        return r(b, n, h, 128).transpose(1, 2)
+    if form == "fused qkv":     # a slice of a wider projection
+        return r(b, n, h + 3, 128)[:, :, 2:2 + h].transpose(1, 2)
+    if form == "every other token":
+        return r(b, h, 2 * n, 128)[:, :, ::2]
+    if form == "one head's rows":
+        return r(b, 1, n, 128).expand(b, h, n, 128)
+    if form == "misaligned":
+        return r(b, h, n, 132)[..., 3:131]
+    if form == "float32":
+        return torch.randn(b, h, n, 128, generator=g, device=dev)
+    if form == "broadcast batch":
+        return r(1, h, n, 128)
+    raise ValueError(form)
+
+
+KERNEL = ["heads first", "tokens first", "fused qkv", "every other token", "one head's rows"]
+TORCH = ["misaligned", "float32", "broadcast batch"]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("form", KERNEL + TORCH)
+@pytest.mark.parametrize("b,h,n", [(1, 8, 1), (2, 3, 15), (1, 8, 64), (3, 2, 65), (1, 1, 300)])
+def test_growing_layer_append(gpu, form, b, h, n, dtype):
+    layer = kv.GrowingLayer()
+    first = rows("heads first", b, h, 7, dtype, gpu, 1)
+    layer.update(first, -first)
+    layer.kbuf[:, :, 7:] = 5.0
+    layer.vbuf[:, :, 7:] = 6.0
+    k, v = rows(form, b, h, n, dtype, gpu, 2), rows("tokens first", b, h, n, dtype, gpu, 3)
+    want_k, want_v = layer.kbuf.clone(), layer.vbuf.clone()
+    want_k[:, :, 7:7 + n] = k
+    want_v[:, :, 7:7 + n] = v
+    assert kv.rows_ok(k, layer.kbuf, n) == (form in KERNEL or form == "broadcast batch")
+    layer.update(k, v)
+    assert layer.n == 7 + n
+    assert torch.equal(layer.kbuf, want_k) and torch.equal(layer.vbuf, want_v)
+
+
+def test_append_under_autograd_stays_with_torch(gpu):
+    layer = kv.GrowingLayer()
+    k = torch.randn(1, 2, 5, 128, device=gpu, dtype=torch.float16, requires_grad=True)
+    assert not kv.rows_ok(k, k.detach(), 5)
+    layer.update(k, k)
+    layer.keys.float().sum().backward()
+    assert torch.equal(k.grad, torch.ones_like(k))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("form", [f for f in KERNEL + TORCH if f != "broadcast batch"])
+@pytest.mark.parametrize("layers,P,n", [(1, 16, 1), (3, 64, 65), (70, 16, 37)])
+def test_paged_append(gpu, form, layers, P, n, dtype):
+    """PagedKV.append (every layer in one launch; 70 layers take two) from a page that is partly full."""
+    h = 3
+    cache = paged.PagedKV(layers, h, 12, P, dtype=dtype, device=gpu)
+    cache.table.free.reverse()
+    start = [rows("heads first", 1, h, 5, dtype, gpu, i) for i in range(layers)]
+    cache.append(0, start, start)
+    ks = [rows(form, 1, h, n, dtype, gpu, 100 + i) for i in range(layers)]
+    vs = [rows("tokens first", 1, h, n, dtype, gpu, 300 + i)[0] for i in range(layers)]
+    cache.append(0, ks, vs)
+    for i in range(layers):
+        k, v = cache.gather(i)
+        assert torch.equal(k, torch.cat((start[i], ks[i].to(dtype)), 2)[0])
+        assert torch.equal(v, torch.cat((start[i][0], vs[i]), 1))
+    used = cache.table.token_slots(0)
+    held = torch.zeros(12, P, dtype=torch.bool)
+    held[used[:, 0], used[:, 1]] = True
+    for pool in cache.k_pools + cache.v_pools:  # nothing else was written
+        assert not pool.transpose(1, 2)[~held.to(gpu)].any()
+
+
+@pytest.mark.parametrize("form", KERNEL + ["misaligned", "float32"])
+@pytest.mark.parametrize("b,n", [(1, 40), (3, 17)])
+def test_paged_layer_update(gpu, form, b, n):
+    """A paged cache layer's update writes every sequence's rows with one launch."""
+
+    class Config:
+        num_hidden_layers = 2
+
+        def get_text_config(self, decoder=True):
+            return self
+
+    cache = paged.new_paged_cache(Config(), 40, 16, batch=b)
+    first = rows("heads first", b, 4, 9, torch.float16, gpu, 5)
+    k, v = rows(form, b, 4, n, torch.float16, gpu, 6), rows("tokens first", b, 4, n, torch.float16, gpu, 7)
+    for i in range(2):
+        cache.update(first, first, i)
+    for i in range(2):
+        cache.update(k, v, i)
+    store = paged.state_of(cache).kv
+    for i in range(2):
+        for j in range(b):
+            gk, gv = store.gather(i, j)
+            assert torch.equal(gk, torch.cat((first[j], k[j].half()), 1)) and torch.equal(gv, torch.cat((first[j], v[j]), 1))

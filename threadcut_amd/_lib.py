@@ -27,8 +27,8 @@ TC_MAX_SPLITS = 4096
 TC_DECODE_SHORT_TOKENS = 2048  # caches up to this long: two-wave partial work-groups
 TC_DECODE_SCRATCH_BYTES = 8 << 20  # static scratch of tc_decode_attention_noalloc, per GPU
 
-_DTYPES = {torch.float16: TC_DTYPE_F16, torch.bfloat16: TC_DTYPE_BF16}
-DTYPES = tuple(_DTYPES)  # element types the kernels take
+DTYPE_CODES = {torch.float16: TC_DTYPE_F16, torch.bfloat16: TC_DTYPE_BF16}
+DTYPES = tuple(DTYPE_CODES)  # element types the kernels take
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int
@@ -72,6 +72,9 @@ SIGNATURES = {
     "tc_splice_copy": (_I, [_PP, _PP, _I64P, _I64, _PP, _PP, _I64P, _I, _I, _I, _I, _I, _I64, _I64, _I64,
                             _FP, _P]),
     "tc_paged_rotate_keys": (_I, [_PP, _I, _I64P, _I, _I, _P, _I64, _I, _I, _I, _FP, _P]),
+    "tc_append_rows": (_I, [_P, _I64P, _P, _I64P, _P, _P, _I64P, _I64, _I64, _I, _I, _I64, _I, _I, _P]),
+    "tc_paged_append_rows": (_I, [_PP, _I64P, _PP, _I64P, _PP, _PP, _I64P, _I, _I, _P, _I, _I, _I, _I64, _I, _I,
+                                  _P]),
     "tc_prefill_attention": (_I, [_P, _I64P, _P, _I64P, _P, _I64P, _P, _I64P, _P, _S, _I, _I64, _I64, _I, _I,
                                   _I, _I, _I, _F, _I, _P, _S, _P, _I64P, _P]),
     "tc_prefill_paged_attention": (_I, [_P, _I64P, _P, _P, _I64P, _I, _P, _I64, _P, _I64P, _P, _S, _I, _I64, _I64,
@@ -146,7 +149,7 @@ def check(rc, what):
 
 def dtype_code(t):
     try:
-        return _DTYPES[t]
+        return DTYPE_CODES[t]
     except KeyError:
         raise TypeError(f"threadcut_amd kernels take float16 or bfloat16 tensors, got {t}") from None
 
@@ -177,7 +180,10 @@ def float_array(t):
 
 
 def stream_of(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The device's current stream as a raw handle. (The raw getter skips the Stream object that
+    torch.cuda.current_stream builds, about 2 us a call.)"""
+    index = device.index
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index))
 
 
 def require_gpu(*tensors, what):

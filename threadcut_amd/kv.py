@@ -20,6 +20,7 @@ from transformers import DynamicCache
 from transformers.cache_utils import DynamicLayer
 
 from . import _lib
+from .flash_decode import _on_device
 from .match import Split  # noqa: F401  (re-exported: the splice contract)
 
 HEAD_DIM = 128
@@ -89,6 +90,44 @@ def _splice_layer_torch(kbuf, vbuf, s, inv_freq):
         v = vbuf[..., s.c0:s.c0 + s.c, :].clone()
         kbuf[..., s.a:s.a + s.c, :] = k
         vbuf[..., s.a:s.a + s.c, :] = v
+
+
+def _plain(t):
+    """False for a tensor that torch records or wraps: autograd, a functorch transform, forward mode, a
+    subclass (tracing). Its copies stay torch ops."""
+    return (type(t) is torch.Tensor and not (t.requires_grad and torch.is_grad_enabled())
+            and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0)
+
+
+def rows_ok(t, buf, rows):
+    """True if the row-writing kernels take `t` as `rows` new tokens of the cache buffer or pool `buf`
+    ([*, heads, *, 128]): a plain [batch, heads, rows, 128] view in the buffer's type and device, 16-byte aligned
+    with strides of whole 16-byte chunks, within the launch grid."""
+    sh, st = t.shape, t.stride()
+    return (t.is_cuda and len(sh) == 4 and sh[3] == HEAD_DIM == buf.shape[-1] and sh[2] == rows < 1 << 22
+            and sh[1] == buf.shape[1] and sh[0] < 512 and t.dtype == buf.dtype and t.dtype in _lib.DTYPES
+            and t.get_device() == buf.get_device() and st[3] == 1 and not (st[0] | st[1] | st[2]) & 7
+            and not t.data_ptr() & 15 and _plain(t))
+
+
+def _append_rows(kbuf, vbuf, row0, k, v):
+    """Rows of the new tokens k/v to rows row0 .. of both buffers: one launch (tc_append_rows) for K and V where
+    the kernel takes them, torch's two copies otherwise (host tensors, other types, head dims or broadcasts)."""
+    add, sb = k.shape[-2], kbuf.stride()
+    if (k.is_cuda and add and len(sb) == 4 and kbuf.shape[0] == k.shape[0] and k.shape == v.shape
+            and sb == vbuf.stride() and rows_ok(k, kbuf, add) and rows_ok(v, vbuf, add)):
+        b, h, cap, d = kbuf.shape
+        sk, sv = k.stride(), v.stride()
+        with _on_device(kbuf.device):
+            rc = _lib.load().tc_append_rows(
+                k.data_ptr(), _lib.i64x3(sk[0], sk[1], sk[2]), v.data_ptr(), _lib.i64x3(sv[0], sv[1], sv[2]),
+                kbuf.data_ptr(), vbuf.data_ptr(), _lib.i64x3(sb[0], sb[1], sb[2]), cap, row0, b, h, add, d,
+                _lib.DTYPE_CODES[kbuf.dtype], _lib.stream_of(kbuf.device))
+        if rc:
+            _lib.check(rc, "tc_append_rows")
+        return
+    kbuf[..., row0:row0 + add, :] = k
+    vbuf[..., row0:row0 + add, :] = v
 
 
 def _as4(t):
@@ -322,8 +361,7 @@ class GrowingLayer(DynamicLayer):
         if self.pending is not None:
             _PENDING.pop(self.kbuf.data_ptr(), None)
             k, v = self.pending
-            self.kbuf[..., self.n - 1:self.n, :] = k
-            self.vbuf[..., self.n - 1:self.n, :] = v
+            _append_rows(self.kbuf, self.vbuf, self.n - 1, k, v)
             self.pending = None
 
     def _reserve(self, need, like):
@@ -358,8 +396,7 @@ class GrowingLayer(DynamicLayer):
             self.pending = (key_states, value_states)
             _PENDING[self.kbuf.data_ptr()] = self
         else:
-            self.kbuf[..., self.n:self.n + add, :] = key_states
-            self.vbuf[..., self.n:self.n + add, :] = value_states
+            _append_rows(self.kbuf, self.vbuf, self.n, key_states, value_states)
         self.n += add
         self._view()
         return self.keys, self.values

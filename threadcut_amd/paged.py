@@ -37,7 +37,7 @@ from transformers.cache_utils import DynamicLayer
 
 from . import _lib
 from .flash_decode import HEAD_DIM, _on_device, _plan
-from .kv import rope_table
+from .kv import rope_table, rows_ok
 from .prefill import GROUPS
 
 TILE = 16  # rows per tile-table entry (the decode kernel's tile)
@@ -72,6 +72,11 @@ def _to_device(arr, device):
     """A host numpy array as a device tensor: staged in pinned memory and copied on the
     current stream without a host wait (torch keeps the staging block until the copy ran)."""
     return torch.from_numpy(np.ascontiguousarray(arr)).pin_memory().to(device, non_blocking=True)
+
+
+def _as_batch(t):
+    """[Hkv, n, D] as [1, Hkv, n, D]."""
+    return t if t.dim() == 4 else t.unsqueeze(0)
 
 
 def _addr(a):
@@ -272,12 +277,37 @@ class PagedKV:
         if n == 0:
             return
         idx = _to_device(slots, self.device)
+        if self.layers and self._write_rows(range(self.layers), [_as_batch(t) for t in ks], [_as_batch(t) for t in vs],
+                                            idx):
+            return
         pages, sl = idx[:, 0], idx[:, 1]
         for kp, vp, k, v in zip(self.k_pools, self.v_pools, ks, vs):
             k = k.reshape(self.kv_heads, n, HEAD_DIM)
             v = v.reshape(self.kv_heads, n, HEAD_DIM)
             kp[pages, :, sl] = k.transpose(0, 1).to(self.dtype)
             vp[pages, :, sl] = v.transpose(0, 1).to(self.dtype)
+
+    def _write_rows(self, layers, ks, vs, slots):
+        """New tokens' rows, per layer [B, Hkv, n, D], into the pools' slots (int64 [B, n, 2] of (page, slot) on the
+        device, or [n, 2] for one sequence) with one launch (tc_paged_append_rows). False if the kernel does not
+        take the tensors (another type, strides that differ between layers): nothing is written then."""
+        b, n = (1, slots.shape[0]) if slots.dim() == 2 else slots.shape[:2]
+        k0, v0 = ks[0], vs[0]
+        for i, k, v in zip(layers, ks, vs):
+            if not (k.shape[0] == v.shape[0] == b and k.stride() == k0.stride() and v.stride() == v0.stride()
+                    and rows_ok(k, self.k_pools[i], n) and rows_ok(v, self.v_pools[i], n)):
+                return False
+        pool = self.k_pools[0]
+        with _on_device(self.device):
+            rc = _lib.load().tc_paged_append_rows(
+                _lib.ptr_array([t.data_ptr() for t in ks]), _lib.i64x3(*k0.stride()[:3]),
+                _lib.ptr_array([t.data_ptr() for t in vs]), _lib.i64x3(*v0.stride()[:3]),
+                _lib.ptr_array([self.k_pools[i].data_ptr() for i in layers]),
+                _lib.ptr_array([self.v_pools[i].data_ptr() for i in layers]), self._strides(), pool.shape[0],
+                pool.shape[2], slots.data_ptr(), len(ks), b, self.kv_heads, n, HEAD_DIM, _lib.dtype_code(self.dtype),
+                _lib.stream_of(self.device))
+        _lib.check(rc, "tc_paged_append_rows")
+        return True
 
     def gather(self, layer, b=0):
         """Sequence b's K and V of one layer in logical order, [Hkv, n, D] copies."""
@@ -607,21 +637,25 @@ class PagedCacheState:
         if need > 0:
             for b in range(self.batch):
                 kv.table.reserve(b, need)
+        slots = self.slots_on_device(layer.n, layer.n + add)
+        if add and kv._write_rows([layer.index], [keys], [values], slots):
+            return
         kp, vp = kv.k_pools[layer.index], kv.v_pools[layer.index]
         for b in range(self.batch):
-            sl = self.slots_on_device(b, layer.n, layer.n + add)
+            sl = slots[b]
             kp[sl[:, 0], :, sl[:, 1]] = keys[b].transpose(0, 1).to(kv.dtype)
             vp[sl[:, 0], :, sl[:, 1]] = values[b].transpose(0, 1).to(kv.dtype)
 
-    def slots_on_device(self, b, lo, hi):
-        """(page, slot) of sequence b's positions [lo, hi) on the device; every layer of a
-        step writes the same positions, so the upload is kept for the table version."""
-        key = (self.kv.table.version, b, lo, hi)
+    def slots_on_device(self, lo, hi):
+        """(page, slot) of every sequence's positions [lo, hi), int64 [B, hi - lo, 2] on the device; every
+        layer of a step writes the same positions, so the upload is kept for the table version."""
+        key = (self.kv.table.version, lo, hi)
         hit = self._slots.get(key)
         if hit is None:
             if self._slots and next(iter(self._slots))[0] != key[0]:
                 self._slots.clear()
-            hit = self._slots[key] = _to_device(self.kv.table.token_slots(b)[lo:hi], self.kv.device)
+            slots = np.stack([self.kv.table.token_slots(b)[lo:hi] for b in range(self.batch)])
+            hit = self._slots[key] = _to_device(slots, self.kv.device)
         return hit
 
     def reserve_step_for(self, layer):
