@@ -167,3 +167,12 @@ def test_attention_is_registered():
     assert attention.NAME == "threadcut"
     assert AttentionInterface._global_mapping[attention.NAME] is attention.attention
     assert attention.NAME in AttentionMaskInterface._global_mapping
+
+
+def test_stride_arrays_are_never_written():
+    """i64x3 arrays are shared between calls: a mask's strides leave those of other tensors alone."""
+    from threadcut_amd import _lib, prefill
+
+    prefill._mask_strides(torch.ones(1, 1, 1, dtype=torch.bool))
+    prefill._mask_strides(torch.ones(2, 3, 5, dtype=torch.bool), batch=False)
+    assert list(_lib.i64x3(0, 0, 0)) == [0, 0, 0] and list(_lib.i64x3(15, 5, 1)) == [15, 5, 1]

@@ -45,11 +45,9 @@ def _strides(t, dims, token_dim=None):
     return _lib.i64x3(*st)
 
 
-def _mask_strides(m):
-    """Strides of a [mb, q, n] mask view; keys are contiguous (stride 1)."""
-    st = _strides(m, (0, 1, 2))
-    st[2] = 1
-    return st
+def _mask_strides(m, batch=True):
+    """Strides of a [mb, q, n] mask view; keys are contiguous (stride 1). batch=False: one mask for every row."""
+    return _lib.i64x3(m.stride(0) if batch and m.shape[0] > 1 else 0, m.stride(1) if m.shape[1] > 1 else 0, 1)
 
 
 def num_splits(batch, q_len, n_tokens, q_heads, kv_heads):
@@ -139,9 +137,7 @@ def mask_tiles(mask, q_heads, kv_heads):
     lib = _lib.load()
     nbytes = lib.tc_prefill_tiles_bytes(q, n, mb, q_heads, kv_heads)
     tiles = torch.empty(max(1, nbytes), dtype=torch.uint8, device=mask.device)
-    st = _mask_strides(m)
-    if mb == 1:
-        st[0] = 0
+    st = _mask_strides(m, batch=mb > 1)
     with torch.cuda.device(mask.device):
         rc = lib.tc_prefill_mask_tiles(m.data_ptr(), st, mb, q, n, q_heads, kv_heads, tiles.data_ptr(),
                                        tiles.numel(), _lib.stream_of(mask.device))
