@@ -427,10 +427,11 @@ int tc_prefill_paged_attention(const void* q, const int64_t q_strides[3],
                                void* out, const int64_t out_strides[3], void* stream);
 
 /* Key splits tc_prefill_attention uses with num_splits <= 0 (a negative value
- * is -TC_ERR_*): 1 when the query blocks (128 rows of one KV head each) give
- * every compute unit two work-groups, else enough splits of the keys to do
- * so, merged by a log-sum-exp combine pass. A short chunk on top of a long
- * cache (the engine's prefill after a splice) is the case this covers. */
+ * is -TC_ERR_*): 1 for a prompt (at least half of the keys are the queries'
+ * own) or when the query blocks fill every compute unit, else as many as fill
+ * them (at most 32), merged by a log-sum-exp combine pass. A short chunk on
+ * top of a long cache (the engine's prefill after a splice) is the case this
+ * covers. */
 int tc_prefill_num_splits(int batch, int64_t q_len, int64_t n_tokens, int q_heads, int kv_heads);
 
 /* Workspace bytes of a call with num_splits splits (0 for one split): fp32
