@@ -141,3 +141,28 @@ def test_strided_rows_and_mask_views(gpu, pad):
     prefill.prefill_attention(q, k, v, m, SCALE, out=out[:, :, 2:18])
     check(out[:, :, 2:18], reference(q, k, v, m[:, 0], SCALE), torch.float16)
     assert not out[:, :, :2].any() and not out[:, :, 18:].any()
+
+
+@pytest.mark.parametrize("ql,n,b,off", [(1, 1, 1, 0), (7, 513, 2, 1), (33, 64, 1, 3), (130, 1500, 3, 2), (40, 511, 1, 0),
+                                        (64, 1025, 2, 5)])
+@pytest.mark.parametrize("hq", [8, 16, 32, 64])
+def test_mask_map(gpu, ql, n, b, off, hq):
+    """The tile map of masks at any alignment: full, empty, causal and mixed tiles, rows and keys past the ends."""
+    tokens, T = 128 // (hq // 8), -(-n // 64)
+    g = torch.Generator(device=gpu).manual_seed(n)
+    m = torch.zeros(b, 1, ql, n + off, dtype=torch.bool, device=gpu)[..., off:]
+    m[:] = workloads.causal_mask(ql, n, device=gpu)
+    m[:, :, ql // 2:, : n // 2] = True
+    m[-1, :, :, : n // 3] = False
+    m[0, :, :, -1] |= torch.rand(1, ql, generator=g, device=gpu) < 0.5
+    got = prefill.mask_tiles(m, hq, 8).cpu()
+    pitch = -(-T // 8) * 8
+    got = got.reshape(b, -1, pitch)
+    causal = workloads.causal_mask(ql, n)[0, 0]
+    for i in range(b):
+        for blk in range(got.shape[1]):
+            rows = slice(blk * tokens, min(ql, (blk + 1) * tokens))
+            for t in range(pitch):
+                x, c = m[i, 0, rows, 64 * t:64 * t + 64].cpu(), causal[rows, 64 * t:64 * t + 64]
+                want = 0 if not x.any() else 1 if x.shape[1] == 64 and x.all() else 3 if torch.equal(x, c) else 2
+                assert got[i, blk, t] == want, (i, blk, t)
