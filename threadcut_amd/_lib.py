@@ -91,11 +91,14 @@ SIGNATURES = {
 
 _lock = threading.Lock()
 _lib = None
+# The native call paths (csrc/host/fastcall.cpp, linked against the default library): None until the library is
+# loaded, and while `using` has another build in its place.
+FAST = None
 
 
 def load():
     """The loaded library (loaded once). Raises RuntimeError if it was not built."""
-    global _lib
+    global _lib, FAST
     if _lib is not None:
         return _lib
     with _lock:
@@ -109,7 +112,12 @@ def load():
                 fn = getattr(lib, name)
                 fn.restype = res
                 fn.argtypes = args
-            _lib = lib
+            try:
+                from . import _fast
+            except ImportError as e:
+                raise RuntimeError(f"threadcut_amd: the native call paths (_fast.so) do not load ({e}); build them "
+                                   "with `python -m threadcut_amd.build`.") from e
+            _lib, FAST = lib, _fast
     return _lib
 
 
@@ -128,15 +136,15 @@ def bind(path):
 def using(lib):
     """Within the block the wrappers call `lib` (a library from ``bind``) instead of the
     default build; the default comes back on exit. For measurement runs in one thread."""
-    global _lib
-    saved = load()
+    global _lib, FAST
+    saved = load(), FAST
     with _lock:
-        _lib = lib
+        _lib, FAST = lib, None
     try:
         yield lib
     finally:
         with _lock:
-            _lib = saved
+            _lib, FAST = saved
 
 
 def check(rc, what):
@@ -179,11 +187,14 @@ def float_array(t):
     return (ctypes.c_float * t.numel())(*t.tolist())
 
 
+raw_stream = torch._C._cuda_getCurrentRawStream  # the current stream of a device index, as a whole number
+
+
 def stream_of(device):
     """The device's current stream as a raw handle. (The raw getter skips the Stream object that
     torch.cuda.current_stream builds, about 2 us a call.)"""
     index = device.index
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index))
+    return ctypes.c_void_p(raw_stream(torch.cuda.current_device() if index is None else index))
 
 
 def require_gpu(*tensors, what):

@@ -21,7 +21,7 @@ import torch.nn.functional as F
 from transformers import AttentionInterface
 from transformers.masking_utils import AttentionMaskInterface, sdpa_mask
 
-from . import kv, paged, prefill
+from . import _lib, kv, paged, prefill
 from .flash_decode import decode_append_at, decode_append_into, decode_into, supports as decode_supports
 
 NAME = "threadcut"
@@ -48,10 +48,23 @@ def attention(module, query, key, value, attention_mask, dropout=0.0, scaling=No
         return paged.attention(layer, query, attention_mask, scaling), None
     hkv = key.shape[1]
     g = hq // hkv
+    pending = kv.take_pending(key)
+    fast = _lib.FAST
+    if q == 1 and attention_mask is None and fast is not None and query.is_cuda:
+        # The whole call in native code; None for what it does not take (then as below).
+        stream = _lib.raw_stream(query.get_device())
+        if pending is None:
+            out = fast.decode(query, key, value, scaling, stream)
+        else:
+            out = fast.decode_append(query, pending.kbuf, pending.vbuf, *pending.pending,
+                                     pending.n if pending.device_pos is None else pending.device_pos, scaling, stream)
+        if out is not None:
+            if pending is not None:
+                pending.pending = None
+            return out, None
     if q == 1 and attention_mask is None and not decode_supports(query, key, value):
         # The reference's decode path for calls its GPU kernel does not serve
         # (attention.py:40-42): the g query heads of a KV head as a length-g query.
-        pending = kv.take_pending(key)
         if pending is not None:
             pending.flush()
         out = F.scaled_dot_product_attention(query.reshape(b, hkv, g, d), key, value, scale=scaling)
@@ -59,21 +72,19 @@ def attention(module, query, key, value, attention_mask, dropout=0.0, scaling=No
     if q == 1 and attention_mask is None:
         # [b, 1, hq, d] contiguous is [b, hkv, g, d] with head index h*g + i.
         out = torch.empty((b, 1, hq, d), dtype=query.dtype, device=query.device)
-        layer = kv.take_pending(key)
-        if layer is not None:
+        if pending is not None:
             # GrowingLayer deferred this token's append: write it and attend in one launch.
-            k_new, v_new = layer.pending
-            layer.pending = None
-            if layer.device_pos is not None:  # graph-captured step: the position lives on the device
-                decode_append_at(query.reshape(b, hkv, g, d), layer.kbuf, layer.vbuf, k_new, v_new,
-                                 layer.device_pos, scaling, out.view(b, hkv, g, d))
+            k_new, v_new = pending.pending
+            pending.pending = None
+            if pending.device_pos is not None:  # graph-captured step: the position lives on the device
+                decode_append_at(query.reshape(b, hkv, g, d), pending.kbuf, pending.vbuf, k_new, v_new,
+                                 pending.device_pos, scaling, out.view(b, hkv, g, d))
             else:
-                decode_append_into(query.reshape(b, hkv, g, d), layer.kbuf, layer.vbuf, k_new, v_new, layer.n,
+                decode_append_into(query.reshape(b, hkv, g, d), pending.kbuf, pending.vbuf, k_new, v_new, pending.n,
                                    scaling, out.view(b, hkv, g, d))
         else:
             decode_into(query.reshape(b, hkv, g, d), key, value, scaling, out.view(b, hkv, g, d))
         return out, None
-    pending = kv.take_pending(key)
     if pending is not None:  # a deferred append must land before SDPA reads the cache
         pending.flush()
     is_causal = attention_mask is None and q > 1 and q == key.shape[2]

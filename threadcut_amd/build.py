@@ -10,6 +10,8 @@ Compiles every ``csrc/*.hip`` source with hipcc (and the host-only
 records a per-wave timeline and the prefill kernel per-tile phase stamps
 (measurement only, ``bench.py --only decode-timeline`` and
 ``--only prefill-timeline``).
+``_fast.so`` (``csrc/host/fastcall.cpp``, g++ against torch's headers) holds the
+wrappers' native call paths; it links to the library.
 When the repository's ``tests/c_host/tc_host.c`` is present, it is built too
 (gcc, C99): a host program that drives the library through the C ABI alone.
 Run as ``python -m threadcut_amd.build``.
@@ -20,6 +22,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -27,6 +30,7 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libthreadcut_hip.so")
 BENCH_LIB = os.path.join(HERE, "libthreadcut_bench.so")
 STAMPS_LIB = os.path.join(HERE, "libthreadcut_stamps.so")
+FAST_LIB = os.path.join(HERE, "_fast.so")
 ARCH = "gfx950"
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 C_HOST = os.path.join(os.path.dirname(HERE), "tests", "c_host", "tc_host.c")
@@ -69,6 +73,32 @@ def _link(objs, lib):
     os.replace(tmp, lib)
 
 
+def _compile_fast(obj):
+    """csrc/host/fastcall.cpp against this Python's torch (host code only)."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    system = [x for p in (*include_paths(), sysconfig.get_paths()["include"]) for x in ("-isystem", p)]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *system, "-c", os.path.join(CSRC, "host", "fastcall.cpp"), "-o", obj]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on fastcall.cpp:\n{r.stderr}")
+
+
+def _link_fast(obj):
+    """_fast.so, a Python module that calls the decode library beside it."""
+    import torch
+
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-shared", obj, f"-L{HERE}", "-lthreadcut_hip", f"-L{lib}", "-ltorch_cpu", "-ltorch_python", "-lc10",
+           "-Wl,-rpath,$ORIGIN", "-o", FAST_LIB + ".tmp"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"link failed:\n{r.stderr}")
+    os.replace(FAST_LIB + ".tmp", FAST_LIB)
+
+
 def build(verbose=False):
     """Compile and link both libraries; returns the decode library's path. Always rebuilds."""
     os.makedirs(BUILD, exist_ok=True)
@@ -81,12 +111,15 @@ def build(verbose=False):
     stamp_objs = [os.path.join(BUILD, "stamps", os.path.splitext(os.path.basename(s))[0] + ".o")
                   for s in stamp_sources]
     defines = [()] * (len(sources) + len(bench_sources)) + [("-DTC_DECODE_STAMPS=1", "-DTC_PREFILL_STAMPS=1")] * len(stamp_sources)
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(every))) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(every) + 1)) as ex:
+        fast = ex.submit(_compile_fast, os.path.join(BUILD, "fastcall.o"))
         for src, warn in zip(every, ex.map(_compile, every, objs + stamp_objs, defines)):
             if warn and verbose:
                 print(f"[{os.path.basename(src)}]\n{warn}", file=sys.stderr)
+        fast.result()
     _link(objs[:len(sources)], LIB)
     _link(objs[len(sources):], BENCH_LIB)
+    _link_fast(os.path.join(BUILD, "fastcall.o"))
     # The host-only objects are shared; only the HIP sources differ.
     host_objs = [o for s, o in zip(sources, objs) if s.endswith(".cpp")]
     _link(stamp_objs + host_objs, STAMPS_LIB)

@@ -113,6 +113,10 @@ def rows_ok(t, buf, rows):
 def _append_rows(kbuf, vbuf, row0, k, v):
     """Rows of the new tokens k/v to rows row0 .. of both buffers: one launch (tc_append_rows) for K and V where
     the kernel takes them, torch's two copies otherwise (host tensors, other types, head dims or broadcasts)."""
+    fast = _lib.FAST
+    if fast is not None and kbuf.is_cuda and fast.append_rows(kbuf, vbuf, row0, k, v,
+                                                              _lib.raw_stream(kbuf.get_device())):
+        return
     add, sb = k.shape[-2], kbuf.stride()
     if (k.is_cuda and add and len(sb) == 4 and kbuf.shape[0] == k.shape[0] and k.shape == v.shape
             and sb == vbuf.stride() and rows_ok(k, kbuf, add) and rows_ok(v, vbuf, add)):

@@ -484,6 +484,16 @@ class PagedKV:
         [B, Hkv, D] (or [B, Hkv, 1, D]) go to the slots `reserve_step` took, and q
         attends every key of its sequence including the new one. Returns out
         [B, Hkv, G, D]."""
+        step, fast = getattr(self, "_step", None), _lib.FAST
+        if (fast is not None and split is None and q.is_cuda and step is not None and step[0] == self.table.version
+                and layer in step[1]):
+            # The whole call in native code; None for what it does not take (then as below).
+            tab, cnt, _ = self.device_table()
+            done = fast.paged_append(q, self.k_pools[layer], self.v_pools[layer], tab, cnt, k_new, v_new, out, scale,
+                                     _lib.raw_stream(q.get_device()))
+            if done is not None:
+                step[1].discard(layer)
+                return done
         _lib.require_gpu(q, k_new, v_new, what="PagedKV.decode_append")
         b, hkv, g, d = q.shape
         if b != self.table.batch or hkv != self.kv_heads or d != HEAD_DIM or q.dtype != self.dtype:
@@ -498,7 +508,6 @@ class PagedKV:
                                  "last dim contiguous")
         if kn.shape != (b, hkv, HEAD_DIM) or vn.shape != (b, hkv, HEAD_DIM):
             raise ValueError("PagedKV.decode_append: k_new/v_new must be [B, Hkv, D]")
-        step = getattr(self, "_step", None)
         if step is None or step[0] != self.table.version or layer not in step[1]:
             raise RuntimeError(f"PagedKV.decode_append: layer {layer} has no reserved slot in this step "
                                "(call reserve_step() once per step, then each layer once)")
