@@ -53,7 +53,7 @@ namespace {
 #define TC_DECODE_INTERLEAVE 1  // tc_decode_attention deals tiles round-robin over the splits
 #endif
 #ifndef TC_DECODE_RAGGED_WGS_PER_CU
-#define TC_DECODE_RAGGED_WGS_PER_CU 8  // the same with per-sequence lengths: finer splits balance them
+#define TC_DECODE_RAGGED_WGS_PER_CU 8  // at most, with per-sequence lengths: finer splits balance them
 #endif
 #ifndef TC_DECODE_WGS_PER_CU
 #define TC_DECODE_WGS_PER_CU 1  // partial work-groups per compute unit the split heuristic aims at
@@ -820,9 +820,15 @@ inline int partial_waves(int64_t n_tokens, bool lens, bool paged, bool append, i
 // unit (every work-group then streams the same share of the cache when its
 // tiles are dealt round-robin), but never more splits than a head has
 // wave-tiles and never more than TC_MAX_SPLITS. Ragged batches (per-sequence
-// lengths) aim at TC_DECODE_RAGGED_WGS_PER_CU per unit: short sequences leave
-// their work-groups light, and many small work-groups let the dispatcher
-// balance the rest. The plan does not depend on the work-group shape: a short
+// lengths) aim at 8, 4 or 2 work-groups per unit where a wave of the longest
+// sequence then still has 4.5 tiles, else at 1: short sequences leave their
+// work-groups light, and many small work-groups let the dispatcher balance the
+// rest, but a work-group costs its first round trip, its merge and its partial
+// whatever it reads. At 8 always, four sequences of 2500-5000 tokens took 21.8
+// us (1.2 tiles a wave) against 13.8 at 2; 16 of 2000-4000 35.2 against 30.5 at
+// 4; 8 of 750-1500 17.6 against 11.3 at 1; 2 of 1500-3000 11.6 against 8.6 at
+// 1; 16 of 1k-32k tokens stay at 8 (150 us against 160 at 4, 156 at 16).
+// The plan does not depend on the work-group shape: a short
 // cache read by two-wave work-groups keeps the four-wave plan's splits (its
 // waves then take two tiles each where four-wave ones took one).
 int split_plan(int batch, int kv_heads, int64_t max_tokens, int split_tokens, int ragged, int* S_out, int* T_out) {
@@ -839,8 +845,14 @@ int split_plan(int batch, int kv_heads, int64_t max_tokens, int split_tokens, in
     int cus = 0;
     const int rc = current_device_cus(&cus);
     if (rc != TC_OK) return rc;
-    const int64_t target = static_cast<int64_t>(ragged ? TC_DECODE_RAGGED_WGS_PER_CU : TC_DECODE_WGS_PER_CU) * cus;
     const int64_t per_head = static_cast<int64_t>(batch) * kv_heads;
+    int64_t per_cu = TC_DECODE_WGS_PER_CU;
+    if (ragged) {
+      const int64_t tiles = ceil_div(max_tokens, kWaveIter), splits1 = std::max<int64_t>(1, cus / per_head);
+      per_cu = TC_DECODE_RAGGED_WGS_PER_CU;
+      while (per_cu > 1 && 2 * tiles < 9 * kWaves * splits1 * per_cu) per_cu /= 2;
+    }
+    const int64_t target = per_cu * cus;
     const int64_t max_s = std::max<int64_t>(1, std::min<int64_t>(ceil_div(ceil_div(max_tokens, kWaveIter), kWaves),
                                                         TC_MAX_SPLITS));
     S = std::max<int64_t>(1, std::min<int64_t>((target + per_head / 2) / per_head, max_s));
