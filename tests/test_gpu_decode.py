@@ -394,3 +394,37 @@ def test_interleaved_partials_cover_round_robin_tiles(gpu, n, split):
         want_l = (m[..., 0] + np.log(p.sum(-1)))
         assert np.abs(o[0, :, s].cpu().numpy() - want_o).max() <= 1e-4
         assert np.abs(lse[0, :, s].cpu().numpy() - want_l).max() <= 1e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,hkv,g,n", [(1, 8, 4, 1), (1, 8, 1, 64), (3, 2, 8, 63), (32, 8, 4, 300), (64, 4, 2, 1000),
+                                       (40, 8, 8, 17)])
+def test_one_split_writes_the_combined_result(gpu, b, hkv, g, n, dtype):
+    """A call of one split (at most 64 tokens, or enough sequences) writes its output from the partial kernel: the
+    bits of the partial pass and the combine, into strided outputs, for plain, ragged and appending calls."""
+    gen = torch.Generator(device=gpu).manual_seed(n)
+    q, k, v = (torch.randn(b, hkv, m, 128, generator=gen, device=gpu).to(dtype) for m in (g, n, n))
+    wide = torch.zeros(b, g, hkv, 192, device=gpu, dtype=dtype)
+    out = wide[..., 32:160].transpose(1, 2)
+    plan = flash_decode.DecodePlan(q, k, v, SCALE, out, split=max(64, -(-n // 64) * 64))
+    assert plan.splits == 1
+    plan.run_partial()
+    plan.run_combine()
+    want = out.clone()
+    wide.zero_()
+    plan.run()
+    # The four-wave and the two-wave work-group sum in different orders.
+    assert torch.equal(out, want) or (n <= 2048 and torch.allclose(out.float(), want.float(), rtol=2 ** -7, atol=1e-3))
+    assert not wide[..., :32].any() and not wide[..., 160:].any()
+    lens = torch.randint(0, n + 1, (b,), generator=gen, device=gpu).to(torch.int32)
+    got = flash_decode.decode_attention_batched(q, k, v, SCALE, lens=lens, split=plan.split_tokens)
+    ref = flash_decode.decode_attention_batched(q, k, v, SCALE, lens=lens, split=64)
+    assert torch.allclose(got.float(), ref.float(), rtol=2 ** -7, atol=2e-3)
+    assert not got[lens == 0].any()
+    kn = torch.randn(b, hkv, 128, generator=gen, device=gpu).to(dtype)
+    kc, vc = k.clone(), v.clone()
+    kc[:, :, -1], vc[:, :, -1] = kn, kn
+    ref = flash_decode.decode_attention_batched(q, kc, vc, SCALE)
+    got = flash_decode.decode_append_into(q, k, v, kn, kn, n, SCALE, torch.empty_like(q))
+    assert torch.equal(k, kc) and torch.equal(v, vc)
+    assert torch.allclose(got.float(), ref.float(), rtol=2 ** -7, atol=2e-3)

@@ -71,7 +71,6 @@ namespace {
 constexpr int kHeadDim = 128;
 constexpr int64_t kMaxTokens = int64_t(1) << 29;  // token positions stay 32-bit in the kernel
 constexpr int kWaves = TC_DECODE_WAVES;
-constexpr int kThreads = 64 * kWaves;
 // Short caches (at most TC_DECODE_SHORT_TOKENS tokens, one length for the
 // batch): partial work-groups of two waves over the same splits. A wave then
 // has two tiles where it had one, and the merge of two waves costs less than
@@ -108,7 +107,7 @@ struct PartialArgs {
   int64_t skn_b, skn_h, svn_b, svn_h;
   uint16_t* k_w;
   uint16_t* v_w;
-  // Paged cache (decode_partial_kernel<DT, true, *>): k and v are page pools
+  // Paged cache (decode_partial_kernel<DT, true, ...>): k and v are page pools
   // [pages, H, P, D] with element strides (sk_b, sk_h, sk_t) = (page, head,
   // token). Sequence b's keys are the tiles tile_tab[b * max_tiles + i],
   // i < tiles[b], each {page, first slot, rows, 0}: rows (<= 16) consecutive
@@ -125,6 +124,10 @@ struct PartialArgs {
   // into the head slab of the pools.
   const int32_t* tok_off;
   int64_t tok_pitch;
+  // One split: the result itself, rounded to the element type as the combine
+  // rounds it (null: the partial goes to o_part, lse_part).
+  uint16_t* out;
+  int64_t so_b, so_h, so_g;
 #if TC_DECODE_STAMPS
   // Per wave ((b * heads + h) * splits + split) * waves + wave, 8 words:
   // realtime-clock stamps (100 MHz) at the kernel's start, after the first
@@ -276,8 +279,9 @@ typedef short lds_s4 __attribute__((ext_vector_type(4)));
 constexpr float kLazyMax = 8.f;               // log2 units the running maximum may lag
 
 // APPEND: the kernel attends (and writes) the new token of an append call
-// (a.k_new != null); the other instantiation carries none of that code.
-template <int DT, bool PAGED, bool APPEND, int W>
+// (a.k_new != null); DIRECT: it writes the result (a.out != null), of one
+// split. The other instantiations carry none of that code.
+template <int DT, bool PAGED, bool APPEND, bool DIRECT, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PAGED ? TC_DECODE_WPE_PAGED : TC_DECODE_WPE))) void decode_partial_kernel(const PartialArgs a) {
   using M = DecodeMma<DT>;
   using E = Elem<DT>;
@@ -496,7 +500,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PAGED ? 
 
   if (APPEND && split == 0 && wave == 0) {
     // The appended token as a tile whose only row is token 0 (the buffer
-    // range is one row, so the other rows read zero and are masked).
+    // range is one row, so the other rows read zero and are masked). Before
+    // the wave's own tiles it holds them up: 11.9 against 11.5 us at 10240
+    // tokens, 8.4 against 7.9 at 4000.
     const char* kn = reinterpret_cast<const char*>(a.k_new + b * a.skn_b + h * a.skn_h);
     const char* vn = reinterpret_cast<const char*>(a.v_new + b * a.svn_b + h * a.svn_h);
     const __amdgpu_buffer_rsrc_t rk = make_rsrc(kn, kHeadDim * 2);
@@ -556,24 +562,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PAGED ? 
   // The head's sum over the four lane groups; m is already common to them.
   l = rows_sum(l);
   const int64_t part = (static_cast<int64_t>(b) * a.heads + h) * a.splits + split;
-  if constexpr (W == 1) {
-    // One wave: its accumulator is the split's; lane (g, n) holds dims
-    // 16 bm + 4 g .. + 3 of head n.
-    if (n < a.group) {
-      const float inv = l == 0.f ? 0.f : __builtin_amdgcn_rcpf(l);
-      float* o = a.o_part + (part * a.group + n) * kHeadDim + 4 * g;
-#pragma unroll
-      for (int bm = 0; bm < 8; ++bm)
-        *reinterpret_cast<float4*>(o + 16 * bm) =
-            make_float4(acc[bm][0] * inv, acc[bm][1] * inv, acc[bm][2] * inv, acc[bm][3] * inv);
-      if (g == 0) a.lse_part[part * a.group + n] = (l == 0.f) ? neg_inf() : (m + __builtin_amdgcn_logf(l)) * kLn2;
-    }
-#if TC_DECODE_STAMPS
-    st_merge = st_loop;
-    record();
-#endif
-    return;
-  }
+  static_assert(W > 1, "the waves of a work-group are merged below");
   if (n < a.group) {
 #pragma unroll
     for (int bm = 0; bm < 8; ++bm)
@@ -617,6 +606,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PAGED ? 
     }
     // L >= 1 whenever a token was seen (the maximum contributes exp2(0)).
     const float inv = L == 0.f ? 0.f : __builtin_amdgcn_rcpf(L);
+    if constexpr (DIRECT) {
+      uint16_t* dst = a.out + b * a.so_b + h * a.so_h + hh * a.so_g + d;
+      *reinterpret_cast<uint32_t*>(dst) = E::bits(O0 * inv) | (E::bits(O1 * inv) << 16);
+      continue;
+    }
     *reinterpret_cast<float2*>(o_out + hh * kHeadDim + d) = make_float2(O0 * inv, O1 * inv);
     if (d == 0) l_out[hh] = (L == 0.f) ? neg_inf() : (Mx + __builtin_amdgcn_logf(L)) * kLn2;
   }
@@ -781,22 +775,22 @@ int check_common(int batch, int kv_heads, int group, int head_dim, int dtype) {
 
 inline dim3 partial_grid(const PartialArgs& a, int batch) { return dim3(a.heads, a.splits, batch); }
 
+template <int DT, bool PAGED, bool APPEND, int W>
+void launch_partial_waves(const PartialArgs& a, int batch, hipStream_t stream) {
+  if (a.out)
+    hipLaunchKernelGGL((decode_partial_kernel<DT, PAGED, APPEND, true, W>), partial_grid(a, batch), dim3(64 * W), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL((decode_partial_kernel<DT, PAGED, APPEND, false, W>), partial_grid(a, batch), dim3(64 * W), 0,
+                       stream, a);
+}
+
 template <int DT, bool PAGED>
 void launch_partial_paged(const PartialArgs& a, int batch, int waves, hipStream_t stream) {
-  if (a.k_new) {
-    hipLaunchKernelGGL((decode_partial_kernel<DT, PAGED, true, kWaves>), partial_grid(a, batch), dim3(kThreads), 0,
-                       stream, a);
-    return;
-  }
-  if constexpr (!PAGED) {
-    if (waves == kShortWaves) {
-      hipLaunchKernelGGL((decode_partial_kernel<DT, false, false, kShortWaves>), partial_grid(a, batch),
-                         dim3(64 * kShortWaves), 0, stream, a);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((decode_partial_kernel<DT, PAGED, false, kWaves>), partial_grid(a, batch), dim3(kThreads), 0,
-                     stream, a);
+  if (a.k_new) return launch_partial_waves<DT, PAGED, true, kWaves>(a, batch, stream);
+  if constexpr (!PAGED)
+    if (waves == kShortWaves) return launch_partial_waves<DT, false, false, kShortWaves>(a, batch, stream);
+  launch_partial_waves<DT, PAGED, false, kWaves>(a, batch, stream);
 }
 
 template <int DT>
@@ -810,8 +804,11 @@ hipError_t launch_partial_dt(const PartialArgs& a, int batch, int waves, hipStre
 
 // Waves per partial work-group: two for a short cache with one length for the
 // batch, read by the plain call with its tiles dealt round-robin; else four.
-inline int partial_waves(int64_t n_tokens, bool lens, bool paged, bool append, int interleave) {
-  return (interleave && !lens && !paged && !append && n_tokens <= TC_DECODE_SHORT_TOKENS) ? kShortWaves : kWaves;
+// A whole call (few_tiles) also asks for at most 8 tiles a split: with more,
+// in a batch, four waves are faster (16 sequences of 1000 tokens, 32 tiles a
+// split: 16.8 against 17.7 us; 4 of 1000, 8 tiles: the same).
+inline int partial_waves(int64_t n_tokens, bool lens, bool paged, bool append, int interleave, bool few_tiles) {
+  return (few_tiles && interleave && !lens && !paged && !append && n_tokens <= TC_DECODE_SHORT_TOKENS) ? kShortWaves : kWaves;
 }
 
 // Split plan of a call: S splits of T tokens each (S * T >= n, T a multiple of
@@ -923,7 +920,8 @@ int partial_impl(const void* q_dev, const int64_t q_strides[3], const void* k_de
                  const void* v_dev, const int64_t v_strides[3], const int32_t* lens_dev, int64_t n_tokens, int batch,
                  int kv_heads, int group, int head_dim, int dtype, float scale, int split_tokens, int num_splits,
                  float* o_part_dev, float* lse_part_dev, int interleave, const Append* app, void* stream,
-                 const Paged* paged = nullptr) {
+                 const Paged* paged = nullptr, bool whole_call = false, void* out_dev = nullptr,
+                 const int64_t* out_strides = nullptr) {
   int rc = check_common(batch, kv_heads, group, head_dim, dtype);
   if (rc != TC_OK) return rc;
   if (n_tokens == 0 && num_splits == 0) return TC_OK;  // empty caches: nothing to read
@@ -992,12 +990,17 @@ int partial_impl(const void* q_dev, const int64_t q_strides[3], const void* k_de
   a.page_tokens = paged ? paged->page_tokens : 0;
   a.tok_off = paged ? paged->tok_off : nullptr;
   a.tok_pitch = paged ? paged->tok_pitch : 0;
+  a.out = static_cast<uint16_t*>(out_dev);
+  a.so_b = out_dev ? out_strides[0] : 0;
+  a.so_h = out_dev ? out_strides[1] : 0;
+  a.so_g = out_dev ? out_strides[2] : 0;
 #if TC_DECODE_STAMPS
   a.stamps = g_stamps;
 #endif
 
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int waves = partial_waves(n_tokens, lens_dev != nullptr, paged != nullptr, app != nullptr, interleave);
+  const int waves = partial_waves(n_tokens, lens_dev != nullptr, paged != nullptr, app != nullptr, interleave,
+                                  !whole_call || n_tokens <= int64_t(8) * kWaveIter * num_splits);
   const hipError_t e = dtype == TC_DTYPE_F16 ? launch_partial_dt<TC_DTYPE_F16>(a, batch, waves, s)
                                              : launch_partial_dt<TC_DTYPE_BF16>(a, batch, waves, s);
   return hip_status(e, "decode_partial launch");
@@ -1082,11 +1085,21 @@ int attention_impl(const void* q_dev, const int64_t q_strides[3], const void* k_
     return fail(TC_ERR_WORKSPACE, "workspace of %zu bytes, %zu needed for %d splits", workspace_bytes, need, S);
   float* o_part = static_cast<float*>(workspace_dev);
   float* lse_part = S > 0 ? o_part + static_cast<size_t>(batch) * kv_heads * S * group * head_dim : nullptr;
+  // One split (many sequences, or at most 64 tokens) needs no combine: the
+  // partial kernel writes the result, bit for bit what the combine would make
+  // of it. 32 sequences of 300 tokens 13.9 -> 10.4 us.
+  const bool direct = S == 1;
+  if (direct) {
+    if (!out_dev) return fail(TC_ERR_INVALID_ARGUMENT, "null tensor pointer");
+    if (!aligned16(out_dev)) return fail(TC_ERR_ALIGNMENT, "out base pointer must be 16-byte aligned");
+    if ((rc = check_strides("out", out_strides, 3)) != TC_OK) return rc;
+  }
   if (S > 0) {
     // Splits here are internal, so their tiles are dealt round-robin (the merged result is the same).
     rc = partial_impl(q_dev, q_strides, k_dev, k_strides, v_dev, v_strides, lens_dev, n_tokens, batch, kv_heads, group,
-                      head_dim, dtype, scale, t, S, o_part, lse_part, TC_DECODE_INTERLEAVE, app, stream, paged);
-    if (rc != TC_OK) return rc;
+                      head_dim, dtype, scale, t, S, o_part, lse_part, TC_DECODE_INTERLEAVE, app, stream, paged,
+                      true, direct ? out_dev : nullptr, out_strides);
+    if (rc != TC_OK || direct) return rc;
   }
   return tc_decode_combine(o_part, lse_part, batch, kv_heads, group, head_dim, S, out_dev, out_strides, dtype, stream);
 }
