@@ -4,11 +4,11 @@
 // SDPA of q [b, hq, L, d] against repeat_kv(k), repeat_kv(v) (each KV head
 // expanded g = hq/hkv times) with the boolean attention mask, or is_causal
 // when there is no mask and L == n; output transposed to [b, L, hq, d].
-// Here the KV heads are never expanded: a work-group owns 128 query rows that
-// are (query token, query head of the group) pairs of ONE KV head, so every
+// Here the KV heads are never expanded: a work-group owns 64 or 128 query rows
+// (Shape; plan() says which shape a call takes) that are (query token, query head of the group) pairs of ONE KV head, so every
 // K/V tile it stages in LDS is read once and shared by the g heads.
 //
-// Per 64-key tile, each wave (32 query rows) computes
+// Per tile, each wave (32 query rows, 32 or 64 of the tile's keys) computes
 //   S^T = K . Q^T   with v_mfma_f32_32x32x16: A = K rows from LDS, B = Q^T
 //                   from registers; lane l then holds 16 of the 32 keys of
 //                   each 32-key half for query row l%32 (the other 16 sit in
@@ -918,8 +918,8 @@ void launch_combine(const PrefillArgs& a, dim3 grid, int hq_total, hipStream_t s
 // The classes of eight tiles (512 keys) of one query block: a thread reads 16
 // keys of every eighth row, 16 bytes at any alignment, and keeps three flags;
 // ballots and LDS join the 32 threads of a tile. Bound: the mask's bytes, read
-// once. (One wave a tile, a byte a lane and row, took 23 us for 2048 x 9764,
-// this 4.6.)
+// once. (One wave a tile, a byte a lane and row, took 23-26 us for 2048 x 9764;
+// this 4.6 on a mask in cache, 7.3 on one just written.)
 constexpr int kMapKeys = 512;
 __global__ __launch_bounds__(256) void mask_tiles_kernel(const uint8_t* mask, int64_t sm_b, int64_t sm_q, int64_t q_len,
                                                          int64_t n, int tokens, int64_t nblk, int64_t pitch,

@@ -3,9 +3,9 @@
 Drop-in for the prefill branch of threadcut/attention.py:43-46, which expands
 every KV head g = Hq/Hkv times (``repeat_kv``, attention.py:25-27) and runs
 SDPA with the boolean mask or ``is_causal``. ``tc_prefill_attention`` reads
-the unexpanded K/V instead: a work-group owns 64 query rows of one KV head
-(64/g tokens × its g query heads), stages each 64-key tile of K and V in LDS
-once for all of them and runs QKᵀ and PV on the matrix cores with an fp32
+the unexpanded K/V instead: a work-group owns 64 or 128 query rows of one KV
+head (rows/g tokens × its g query heads), stages each tile of 64 or 128 keys of
+K and V in LDS once for all of them and runs QKᵀ and PV on the matrix cores with an fp32
 online softmax. This module checks tensors and passes pointers, strides and
 the current stream.
 """
