@@ -86,6 +86,17 @@ def test_split_counts(gpu, hq, hkv, ql, n, splits):
         check(out, reference(q, k, v, vis, SCALE), torch.float16)
 
 
+@pytest.mark.parametrize("hq,hkv", [(3, 3), (6, 3), (20, 5), (56, 7)])
+@pytest.mark.parametrize("b,ql", [(1, 2), (2, 9), (1, 77)])
+def test_combine_of_odd_heads_and_rows(gpu, hq, hkv, b, ql):
+    """Eight rows of one KV head per combine work-group: the last group of a head is partly empty."""
+    n = 2500
+    q, k, v = workloads.prefill_inputs(ql, batch=b, q_len=ql, n=n, q_heads=hq, kv_heads=hkv, dtype=torch.float16, device=gpu)
+    m, vis = masks("chunk", ql, n, b, gpu, n)
+    assert prefill.num_splits(b, ql, n, hq, hkv) > 1
+    check(prefill.prefill_attention(q, k, v, m, SCALE, False), reference(q, k, v, vis, SCALE), torch.float16)
+
+
 @pytest.mark.parametrize("hq,hkv,ql,n", [(16, 8, 200, 257), (32, 8, 5, 3000), (32, 8, 100, 5000), (32, 8, 1100, 1100)])
 @pytest.mark.parametrize("P", [16, 48, 64])
 def test_paged_shapes(gpu, hq, hkv, ql, n, P):
