@@ -4,7 +4,8 @@ kernels do not take (misaligned, another type, a broadcast batch) go through tor
 import pytest
 import torch
 
-from threadcut_amd import kv, paged
+from threadcut_amd import _lib, kv, paged
+from threadcut_amd.match import Split
 
 pytestmark = pytest.mark.gpu
 
@@ -64,6 +65,96 @@ def test_append_under_autograd_stays_with_torch(gpu):
     assert torch.equal(k.grad, torch.ones_like(k))
 
 
+class Config:
+    num_hidden_layers = 2
+
+    def get_text_config(self, decoder=True):
+        return self
+
+
+STORES = ["layer", "layer, Python path", "slab", "slab, Python path", "pools", "paged layer"]
+
+
+class Store:
+    """Two heads of one sequence behind one of the caches that appends reach: rows in, cut to n tokens, and the
+    tensor the cache reads its K from."""
+
+    def __init__(self, kind, gpu, monkeypatch):
+        self.kind = kind
+        if "Python path" in kind:
+            _lib.load()
+            monkeypatch.setattr(_lib, "FAST", None)
+        if kind == "pools":
+            self.kv = paged.PagedKV(1, 2, 4, 16, device=gpu)
+        elif kind == "paged layer":
+            self.cache = paged.new_paged_cache(Config(), 8, 16)
+            self.layer = self.cache.layers[0]
+        else:
+            self.layer = kv.new_cache(Config(), slab=kind.startswith("slab")).layers[0]
+
+    def append(self, k, v):
+        if self.kind == "pools":
+            self.kv.append(0, [k], [v])
+        else:
+            self.layer.update(k, v)
+
+    def cut(self, n):
+        if self.kind == "pools":
+            self.kv.prune(0, Split(n, self.kv.length(), 0), None)
+        elif self.kind == "paged layer":
+            store = paged.state_of(self.cache).kv
+            store.table.prune(0, n, store.length(), 0)
+            self.layer.n = n
+        else:
+            self.layer.crop(n)
+
+    def keys(self):
+        if self.kind not in ("pools", "paged layer"):
+            return self.layer.keys[0]
+        store = self.kv if self.kind == "pools" else paged.state_of(self.cache).kv
+        return store.k_pools[0][int(store.table.token_slots(0)[0, 0])]
+
+
+@pytest.mark.parametrize("kind", STORES)
+def test_append_over_rows_that_autograd_tracks(gpu, monkeypatch, kind):
+    """Plain rows written over tracked ones cut those off: no gradient reaches the rows that are gone."""
+    s = Store(kind, gpu, monkeypatch)
+    k = torch.randn(1, 2, 5, 128, device=gpu, dtype=torch.float16, requires_grad=True)
+    s.append(k, k.detach())
+    s.cut(3)
+    s.append(rows("heads first", 1, 2, 2, torch.float16, gpu, 1), rows("heads first", 1, 2, 2, torch.float16, gpu, 2))
+    s.keys().float().sum().backward()
+    want = torch.zeros_like(k)
+    want[:, :, :3] = 1
+    assert torch.equal(k.grad, want)
+
+
+@pytest.mark.parametrize("kind", STORES)
+def test_append_tells_autograd_of_the_write(gpu, monkeypatch, kind):
+    """Rows that an operation saved for its backward and an append has overwritten: backward refuses them."""
+    s = Store(kind, gpu, monkeypatch)
+    s.append(rows("heads first", 1, 2, 5, torch.float16, gpu, 1), rows("heads first", 1, 2, 5, torch.float16, gpu, 2))
+    w = torch.ones(128, device=gpu, dtype=torch.float16, requires_grad=True)
+    y = (s.keys() * w).sum()
+    s.cut(3)
+    with torch.no_grad():
+        s.append(rows("heads first", 1, 2, 2, torch.float16, gpu, 3), rows("heads first", 1, 2, 2, torch.float16, gpu, 4))
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward()
+
+
+@pytest.mark.parametrize("kind", STORES)
+def test_append_outside_inference_mode_keeps_its_refusal(gpu, monkeypatch, kind):
+    """A cache made in inference mode takes rows there and, like any inference tensor, nowhere else."""
+    with torch.inference_mode():
+        s = Store(kind, gpu, monkeypatch)
+        x = rows("heads first", 1, 2, 5, torch.float16, gpu, 1)
+        s.append(x, x)
+        s.append(x, x)
+    with pytest.raises(RuntimeError, match="inference tensor"):
+        s.append(rows("heads first", 1, 2, 5, torch.float16, gpu, 2), rows("heads first", 1, 2, 5, torch.float16, gpu, 2))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("form", [f for f in KERNEL + TORCH if f != "broadcast batch"])
 @pytest.mark.parametrize("layers,P,n", [(1, 16, 1), (3, 64, 65), (70, 16, 37)])
@@ -92,13 +183,6 @@ def test_paged_append(gpu, form, layers, P, n, dtype):
 @pytest.mark.parametrize("b,n", [(1, 40), (3, 17)])
 def test_paged_layer_update(gpu, form, b, n):
     """A paged cache layer's update writes every sequence's rows with one launch."""
-
-    class Config:
-        num_hidden_layers = 2
-
-        def get_text_config(self, decoder=True):
-            return self
-
     cache = paged.new_paged_cache(Config(), 40, 16, batch=b)
     first = rows("heads first", b, 4, 9, torch.float16, gpu, 5)
     k, v = rows(form, b, 4, n, torch.float16, gpu, 6), rows("tokens first", b, 4, n, torch.float16, gpu, 7)

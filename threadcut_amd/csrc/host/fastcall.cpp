@@ -12,6 +12,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/InferenceMode.h>
 #include <c10/core/impl/DeviceGuardImplInterface.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/Exceptions.h>
@@ -241,7 +242,15 @@ PyObject* paged_append(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
-// append_rows(k_buf, v_buf [b, h, cap, d], row0, k, v [b, h, rows, d], stream) -> bool: new tokens' rows into both buffers.
+// True for a tensor whose in-place copy torch would record or refuse: autograd (a view of a tracked buffer counts),
+// a forward-mode tangent, an inference tensor outside inference mode.
+bool recorded(const at::Tensor& t) {
+  return (c10::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(0).defined() ||
+         (t.is_inference() && !c10::InferenceMode::is_enabled());
+}
+
+// append_rows(k_buf, v_buf [b, h, cap, d], row0, k, v [b, h, rows, d], stream) -> bool: new tokens' rows into both
+// buffers. Autograd is told of the write (the buffers' versions), as torch's copy would tell it.
 PyObject* append_rows(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
   c10::Device dev(c10::DeviceType::CPU);
@@ -250,13 +259,13 @@ PyObject* append_rows(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   int dt;
   if (!kb || !vb || !k || !v || kb->dim() != 4 || k->dim() != 4 || !dtype_code(*kb, &dt)) Py_RETURN_FALSE;
   if (vb->sizes() != kb->sizes() || vb->strides() != kb->strides() || v->sizes() != k->sizes()) Py_RETURN_FALSE;
-  for (const at::Tensor* t : {k, v}) {
-    // Rows that autograd or a functorch transform would record stay torch's copies.
+  for (const at::Tensor* t : {k, v})
     if (!same_type(*kb, *t) || t->size(0) != kb->size(0) || t->size(1) != kb->size(1) || t->size(3) != kHeadDim ||
-        kb->size(3) != kHeadDim || t->stride(3) != 1 || (t->requires_grad() && c10::GradMode::is_enabled()) ||
-        t->_fw_grad(0).defined())
+        kb->size(3) != kHeadDim || t->stride(3) != 1)
       Py_RETURN_FALSE;
-  }
+  // Writes that autograd or a functorch transform would record stay torch's copies.
+  for (const at::Tensor* t : {kb, vb, k, v})
+    if (recorded(*t)) Py_RETURN_FALSE;
   if (c10::impl::tls_local_dispatch_key_set().included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) Py_RETURN_FALSE;
   const int64_t row0 = PyLong_AsLongLong(a[2]);
   void* stream = raw_stream(a[5]);
@@ -270,6 +279,8 @@ PyObject* append_rows(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
                       kHeadDim, dt, stream);
   Py_END_ALLOW_THREADS
   if (rc != TC_OK) Py_RETURN_FALSE;
+  if (!kb->is_inference()) kb->unsafeGetTensorImpl()->bump_version();
+  if (!vb->is_inference()) vb->unsafeGetTensorImpl()->bump_version();
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }

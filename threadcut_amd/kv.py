@@ -16,6 +16,7 @@ without contraction, so shifted keys match the reference's fp32 op sequence
 bit for bit.
 """
 import torch
+from torch.autograd.graph import increment_version
 from transformers import DynamicCache
 from transformers.cache_utils import DynamicLayer
 
@@ -93,21 +94,24 @@ def _splice_layer_torch(kbuf, vbuf, s, inv_freq):
 
 
 def _plain(t):
-    """False for a tensor that torch records or wraps: autograd, a functorch transform, forward mode, a
-    subclass (tracing). Its copies stay torch ops."""
+    """False for a tensor whose in-place copy torch records or refuses: autograd (a view of a tracked buffer counts),
+    a functorch transform, forward mode, a subclass, an inference tensor outside inference mode. Its copies stay
+    torch ops."""
     return (type(t) is torch.Tensor and not (t.requires_grad and torch.is_grad_enabled())
-            and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0)
+            and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
+            and not (t.is_inference() and not torch.is_inference_mode_enabled()))
 
 
 def rows_ok(t, buf, rows):
     """True if the row-writing kernels take `t` as `rows` new tokens of the cache buffer or pool `buf`
     ([*, heads, *, 128]): a plain [batch, heads, rows, 128] view in the buffer's type and device, 16-byte aligned
-    with strides of whole 16-byte chunks, within the launch grid."""
+    with strides of whole 16-byte chunks, within the launch grid, and a buffer that autograd does not track. Whoever
+    launches such a kernel tells autograd of the write (increment_version), as torch's copy would."""
     sh, st = t.shape, t.stride()
     return (t.is_cuda and len(sh) == 4 and sh[3] == HEAD_DIM == buf.shape[-1] and sh[2] == rows < 1 << 22
             and sh[1] == buf.shape[1] and sh[0] < 512 and t.dtype == buf.dtype and t.dtype in _lib.DTYPES
             and t.get_device() == buf.get_device() and st[3] == 1 and not (st[0] | st[1] | st[2]) & 7
-            and not t.data_ptr() & 15 and _plain(t))
+            and not t.data_ptr() & 15 and _plain(t) and _plain(buf))
 
 
 def _append_rows(kbuf, vbuf, row0, k, v):
@@ -129,6 +133,7 @@ def _append_rows(kbuf, vbuf, row0, k, v):
                 _lib.DTYPE_CODES[kbuf.dtype], _lib.stream_of(kbuf.device))
         if rc:
             _lib.check(rc, "tc_append_rows")
+        increment_version((kbuf, vbuf))
         return
     kbuf[..., row0:row0 + add, :] = k
     vbuf[..., row0:row0 + add, :] = v

@@ -32,6 +32,7 @@ import weakref
 import numpy as np
 import torch
 import torch.nn.functional as F
+from torch.autograd.graph import increment_version
 from transformers import DynamicCache
 from transformers.cache_utils import DynamicLayer
 
@@ -307,6 +308,7 @@ class PagedKV:
                 pool.shape[2], slots.data_ptr(), len(ks), b, self.kv_heads, n, HEAD_DIM, _lib.dtype_code(self.dtype),
                 _lib.stream_of(self.device))
         _lib.check(rc, "tc_paged_append_rows")
+        increment_version([pools[i] for i in layers for pools in (self.k_pools, self.v_pools)])
         return True
 
     def gather(self, layer, b=0):
