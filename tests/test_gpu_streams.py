@@ -10,6 +10,8 @@ result is checked against the oracle: decode and fused-append decode (float64
 closed form, 2e-3), prefill (float64 closed form, 2e-3), the GrowingLayer
 splice (bit-exact) and the paged prune + decode.
 """
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -19,7 +21,7 @@ from oracle import prefill as opf
 from oracle import splice as osp
 from threadcut_amd import flash_decode, kv, prefill, workloads
 from threadcut_amd.match import Split
-from threadcut_amd.paged import PagedKV
+from threadcut_amd.paged import PagedKV, new_paged_cache, state_of
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +133,102 @@ def test_paged_prune_and_decode_on_a_side_stream(gpu):
     assert np.array_equal(vg.cpu().numpy().view(np.uint16), vw.view(np.uint16))
     want = od.attention_f64(qh.float().numpy(), kw[None].astype(np.float32), vw[None].astype(np.float32), D ** -0.5)
     assert np.abs(out.float().cpu().numpy() - want).max() <= 2e-3
+
+
+def running_stream(gpu):
+    """A side stream whose work runs now: streams share a few hardware queues, and one behind a spinning stream's
+    would wait for it whatever the code under test does."""
+    for _ in range(8):
+        side = torch.cuda.Stream(device=gpu)
+        with torch.cuda.stream(side):
+            torch.zeros(1, device=gpu)
+        for _ in range(50):
+            if side.query():
+                return side
+            time.sleep(0.001)
+    raise AssertionError("every side stream waits for the spinning one")
+
+
+def zeros_to_reuse(shape, dtype, gpu):
+    """Zeroed device memory handed back to the current stream's pool: the next tensor of this size holds zeros until
+    it is written."""
+    torch.zeros(shape, dtype=dtype, device=gpu)
+
+
+def test_a_mask_map_is_waited_for_by_other_streams(gpu):
+    """The tile map of a mask is built on the stream of its first call; a call on another stream that meets the same
+    mask waits for it."""
+    b, hq, hkv, ql, n = 1, 32, 8, 200, 900
+    q, k, v = (rnd(s, i).to(gpu) for i, s in enumerate(((b, hq, ql, D), (b, hkv, n, D), (b, hkv, n, D))))
+    m = (torch.arange(n, device=gpu)[None, :] <= torch.arange(ql, device=gpu)[:, None] + (n - ql))[None, None]
+    m[..., 5:90] = False
+    want = prefill.prefill_attention(q, k, v, m.clone(), D ** -0.5)
+    map_bytes = prefill.mask_tiles(m.clone(), hq, hkv).numel()
+    first = torch.cuda.Stream(device=gpu)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        zeros_to_reuse(map_bytes, torch.uint8, gpu)  # every tile of such a map would be skipped
+        torch.cuda._sleep(SPIN)
+        a = prefill.prefill_attention(q, k, v, m, D ** -0.5)
+    with torch.cuda.stream(running_stream(gpu)):
+        got = prefill.prefill_attention(q, k, v, m, D ** -0.5)
+        again = prefill.prefill_attention(q, k, v, m, D ** -0.5)
+    assert not first.query(), "the spin ended before the calls were enqueued"
+    torch.cuda.synchronize()
+    assert torch.equal(a, want) and torch.equal(got, want) and torch.equal(again, want)
+
+
+class TwoLayers:
+    num_hidden_layers = 2
+
+    def get_text_config(self, decoder=True):
+        return self
+
+
+def test_paged_slots_are_waited_for_by_other_streams(gpu):
+    """The slot list of a chunk is uploaded by the first layer's append; another layer's append on another stream
+    waits for it."""
+    n = 40
+    k = [rnd((1, 8, n, D), i).to(gpu) for i in range(2)]
+    cache = new_paged_cache(TwoLayers(), 8, 16)
+    for i in range(2):
+        cache.update(k[i][:, :, :16], k[i][:, :, :16], i)
+    first = torch.cuda.Stream(device=gpu)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        zeros_to_reuse((1, n, 2), torch.int64, gpu)  # every row of such a list would go to slot 0 of page 0
+        torch.cuda._sleep(SPIN)
+        cache.update(k[0], k[0], 0)
+    with torch.cuda.stream(running_stream(gpu)):
+        cache.update(k[1], k[1], 1)
+    assert not first.query(), "the spin ended before the calls were enqueued"
+    torch.cuda.synchronize()
+    for i in range(2):
+        gk, gv = state_of(cache).kv.gather(i)
+        want = torch.cat((k[i][0, :, :16], k[i][0]), 1)
+        assert torch.equal(gk, want) and torch.equal(gv, want)
+
+
+def test_paged_tables_are_waited_for_by_other_streams(gpu):
+    """The tile table and the token offsets are uploaded by the first call that reads them; decode and prefill calls
+    on another stream wait for them."""
+    n = 300
+    k, q, qp = rnd((8, n, D), 1).to(gpu), rnd((1, 8, 4, D), 2).to(gpu), rnd((1, 32, 20, D), 3).to(gpu)
+    want = None
+    for spin in (0, SPIN):
+        cache = PagedKV(1, 8, 24, 16, device=gpu)
+        cache.append(0, [k], [k])
+        first = torch.cuda.Stream(device=gpu)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(first):
+            if spin:
+                torch.cuda._sleep(spin)
+            got = [cache.decode(0, q, D ** -0.5), cache.prefill(0, qp, D ** -0.5)]
+        if spin:
+            with torch.cuda.stream(running_stream(gpu)):
+                got += [cache.decode(0, q, D ** -0.5), cache.prefill(0, qp, D ** -0.5)]
+            assert not first.query(), "the spin ended before the calls were enqueued"
+        torch.cuda.synchronize()
+        want = want or got
+        for i, x in enumerate(got):
+            assert torch.equal(x, want[i % 2])

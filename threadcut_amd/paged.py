@@ -253,7 +253,7 @@ class PagedKV:
         # The pools' own device, with its index ("cuda" alone names the current device).
         self.device = self.k_pools[0].device if self.k_pools else torch.device(
             "cuda", torch.cuda.current_device() if dev.index is None else dev.index)
-        self._dev_table = None  # (version, table, tiles, max_tiles)
+        self._dev_table = None  # (version, (table, tiles) on the device, max_tiles)
 
     @property
     def layers(self):
@@ -327,9 +327,10 @@ class PagedKV:
         ver = self.table.version
         if self._dev_table is None or self._dev_table[0] != ver:
             tab, cnt = self.table.tile_table()
-            self._dev_table = (ver, _to_device(tab, self.device), _to_device(cnt, self.device),
+            self._dev_table = (ver, _lib.Resident(_to_device(tab, self.device), _to_device(cnt, self.device)),
                                tab.shape[1])
-        return self._dev_table[1:]
+        _, tables, max_tiles = self._dev_table
+        return (*tables.get(), max_tiles)
 
     def device_offsets(self):
         """(token offsets int32 [B, pitch], pitch) on the device: the byte offset of each logical
@@ -339,8 +340,9 @@ class PagedKV:
         if getattr(self, "_dev_off", None) is None or self._dev_off[0] != ver:
             st = self.k_pools[0].stride()
             off = self.table.token_offsets(st[0] * 2, st[2] * 2)
-            self._dev_off = (ver, _to_device(off, self.device), off.shape[1])
-        return self._dev_off[1:]
+            self._dev_off = (ver, _lib.Resident(_to_device(off, self.device)), off.shape[1])
+        _, offsets, pitch = self._dev_off
+        return (*offsets.get(), pitch)
 
     def prefill(self, layer, query, scale, mask=None, causal=False, out=None):
         """The prefill branch of threadcut/attention.py:43-46 over the pools: query
@@ -666,8 +668,8 @@ class PagedCacheState:
             if self._slots and next(iter(self._slots))[0] != key[0]:
                 self._slots.clear()
             slots = np.stack([self.kv.table.token_slots(b)[lo:hi] for b in range(self.batch)])
-            hit = self._slots[key] = _to_device(slots, self.kv.device)
-        return hit
+            hit = self._slots[key] = _lib.Resident(_to_device(slots, self.kv.device))
+        return hit.get()[0]
 
     def reserve_step_for(self, layer):
         """A decode step's slot per sequence: reserved by the first layer of the step."""

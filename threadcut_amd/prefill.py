@@ -130,7 +130,7 @@ def mask_tiles(mask, q_heads, kv_heads):
     key = (mask._version, tuple(mask.shape), tuple(mask.stride()), mask.data_ptr(), q_heads, kv_heads)
     c = _tile_cache
     if c is not None and c[0]() is mask and c[1] == key:
-        return c[2]
+        return c[2].get()[0]
     m = mask[:, 0]
     mb = m.shape[0] if m.shape[0] > 1 and m.stride(0) != 0 else 1
     q, n = m.shape[1], m.shape[2]
@@ -142,5 +142,5 @@ def mask_tiles(mask, q_heads, kv_heads):
         rc = lib.tc_prefill_mask_tiles(m.data_ptr(), st, mb, q, n, q_heads, kv_heads, tiles.data_ptr(),
                                        tiles.numel(), _lib.stream_of(mask.device))
     _lib.check(rc, "tc_prefill_mask_tiles")
-    _tile_cache = (weakref.ref(mask), key, tiles)
+    _tile_cache = (weakref.ref(mask), key, _lib.Resident(tiles))
     return tiles
