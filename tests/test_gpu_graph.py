@@ -19,7 +19,7 @@ import torch
 from transformers import AutoModelForCausalLM, Qwen3Config
 
 from oracle import decode as od
-from threadcut_amd import attention, flash_decode, kv, workloads
+from threadcut_amd import attention, flash_decode, kv, prefill, workloads
 from threadcut_amd.graph import DecodeGraph
 
 pytestmark = pytest.mark.gpu
@@ -251,3 +251,26 @@ def test_decode_graph_refuses_changes_outside_the_graph(model):
     assert cache.get_seq_length() == 27
     out = model(input_ids=torch.tensor([[9]], device=dev), past_key_values=cache, use_cache=True).logits
     assert bool(torch.isfinite(out).all()) and cache.get_seq_length() == 28
+
+
+def test_captured_prefill_follows_its_mask(gpu):
+    """A captured prefill call classifies its mask's tiles on every replay: a mask written anew in place counts, also
+    where an eager call had met the mask before the capture, and eager calls in between keep theirs."""
+    ql, n = 200, 900
+    q, k, v = workloads.prefill_inputs(3, q_len=ql, n=n, device=gpu)
+    causal = workloads.causal_mask(ql, n, device=gpu)
+    masks = [(causal & (torch.arange(n, device=gpu) >= lo)).contiguous() for lo in (0, 130, 400)]
+    want = [prefill.prefill_attention(q, k, v, m.clone(), SCALE) for m in masks]
+    m = masks[0].clone()
+    assert torch.equal(prefill.prefill_attention(q, k, v, m, SCALE), want[0])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = prefill.prefill_attention(q, k, v, m, SCALE)
+    for r in (1, 2, 0, 2, 1):
+        print(f"case: mask {r}", flush=True)
+        m.copy_(masks[r])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[r])
+        assert torch.equal(prefill.prefill_attention(q, k, v, m, SCALE), want[r])
+        assert torch.equal(prefill.prefill_attention(q, k, v, masks[0], SCALE), want[0])

@@ -121,6 +121,8 @@ def prefill_attention(query, key, value, attention_mask=None, scale=None, is_cau
 # The tile map of the last mask seen. transformers builds one mask per forward
 # pass and hands the same tensor to every layer, so the map is built once per
 # pass; it is rebuilt when the mask object, its version or the geometry change.
+# A captured call builds its own: a replay must not read a map that it did not
+# make, of the mask as it was before.
 _tile_cache = None
 
 
@@ -128,8 +130,8 @@ def mask_tiles(mask, q_heads, kv_heads):
     """uint8 tile map of a bool mask [b|1, 1, q, n] (``tc_prefill_mask_tiles``), cached per mask."""
     global _tile_cache
     key = (mask._version, tuple(mask.shape), tuple(mask.stride()), mask.data_ptr(), q_heads, kv_heads)
-    c = _tile_cache
-    if c is not None and c[0]() is mask and c[1] == key:
+    c, captured = _tile_cache, torch.cuda.is_current_stream_capturing()
+    if c is not None and not captured and c[0]() is mask and c[1] == key:
         return c[2].get()[0]
     m = mask[:, 0]
     mb = m.shape[0] if m.shape[0] > 1 and m.stride(0) != 0 else 1
@@ -142,5 +144,6 @@ def mask_tiles(mask, q_heads, kv_heads):
         rc = lib.tc_prefill_mask_tiles(m.data_ptr(), st, mb, q, n, q_heads, kv_heads, tiles.data_ptr(),
                                        tiles.numel(), _lib.stream_of(mask.device))
     _lib.check(rc, "tc_prefill_mask_tiles")
-    _tile_cache = (weakref.ref(mask), key, _lib.Resident(tiles))
+    if not captured:
+        _tile_cache = (weakref.ref(mask), key, _lib.Resident(tiles))
     return tiles
