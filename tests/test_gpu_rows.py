@@ -155,6 +155,32 @@ def test_append_outside_inference_mode_keeps_its_refusal(gpu, monkeypatch, kind)
         s.append(rows("heads first", 1, 2, 5, torch.float16, gpu, 2), rows("heads first", 1, 2, 5, torch.float16, gpu, 2))
 
 
+@pytest.mark.parametrize("kind", STORES)
+def test_append_is_recorded_by_tracing(gpu, monkeypatch, kind):
+    """torch.jit.trace, make_fx and torch.compile record the write: what they return follows new inputs."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    def f(k):
+        s = Store(kind, gpu, monkeypatch)
+        s.append(k, k)
+        return s.keys()[:, :5].clone()
+
+    a, b = (rows("heads first", 1, 2, 5, torch.float16, gpu, i) for i in (1, 2))
+    assert torch.equal(f(b), b[0])
+    assert torch.equal(make_fx(f)(a)(b), b[0])
+    with torch.no_grad():
+        assert torch.equal(torch.jit.trace(f, (a,), check_trace=False)(b), b[0])
+    if kind in ("layer", "slab"):  # (the page table is host code, which compilation does not enter)
+        s = Store(kind, gpu, monkeypatch)
+        s.append(a, a)
+
+        def g(k):
+            s.append(k, k)
+            return s.layer.keys.clone()
+
+        assert torch.equal(torch.compile(g, backend="eager", fullgraph=True)(b), torch.cat((a, b), 2))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("form", [f for f in KERNEL + TORCH if f != "broadcast batch"])
 @pytest.mark.parametrize("layers,P,n", [(1, 16, 1), (3, 64, 65), (70, 16, 37)])

@@ -249,6 +249,12 @@ bool recorded(const at::Tensor& t) {
          (t.is_inference() && !c10::InferenceMode::is_enabled());
 }
 
+// True while something sees every operation of this thread: torch.jit.trace, a dispatch mode and a functorch transform
+// each include a dispatch key of their own.
+bool watched() {
+  return !(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty();
+}
+
 // append_rows(k_buf, v_buf [b, h, cap, d], row0, k, v [b, h, rows, d], stream) -> bool: new tokens' rows into both
 // buffers. Autograd is told of the write (the buffers' versions), as torch's copy would tell it.
 PyObject* append_rows(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
@@ -263,10 +269,10 @@ PyObject* append_rows(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (!same_type(*kb, *t) || t->size(0) != kb->size(0) || t->size(1) != kb->size(1) || t->size(3) != kHeadDim ||
         kb->size(3) != kHeadDim || t->stride(3) != 1)
       Py_RETURN_FALSE;
-  // Writes that autograd or a functorch transform would record stay torch's copies.
+  // Writes that autograd, tracing, a dispatch mode or a functorch transform would record stay torch's copies.
   for (const at::Tensor* t : {kb, vb, k, v})
     if (recorded(*t)) Py_RETURN_FALSE;
-  if (c10::impl::tls_local_dispatch_key_set().included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) Py_RETURN_FALSE;
+  if (watched()) Py_RETURN_FALSE;
   const int64_t row0 = PyLong_AsLongLong(a[2]);
   void* stream = raw_stream(a[5]);
   if (PyErr_Occurred()) return nullptr;

@@ -93,12 +93,17 @@ def _splice_layer_torch(kbuf, vbuf, s, inv_freq):
         vbuf[..., s.a:s.a + s.c, :] = v
 
 
+def _watched():
+    """True while torch records every operation: compilation, torch.jit.trace, a dispatch mode (make_fx), a functorch
+    transform, forward mode. Writes stay torch ops then."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0)
+
+
 def _plain(t):
     """False for a tensor whose in-place copy torch records or refuses: autograd (a view of a tracked buffer counts),
-    a functorch transform, forward mode, a subclass, an inference tensor outside inference mode. Its copies stay
-    torch ops."""
+    a subclass, an inference tensor outside inference mode. Its copies stay torch ops."""
     return (type(t) is torch.Tensor and not (t.requires_grad and torch.is_grad_enabled())
-            and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
             and not (t.is_inference() and not torch.is_inference_mode_enabled()))
 
 
@@ -108,7 +113,7 @@ def rows_ok(t, buf, rows):
     with strides of whole 16-byte chunks, within the launch grid, and a buffer that autograd does not track. Whoever
     launches such a kernel tells autograd of the write (increment_version), as torch's copy would."""
     sh, st = t.shape, t.stride()
-    return (t.is_cuda and len(sh) == 4 and sh[3] == HEAD_DIM == buf.shape[-1] and sh[2] == rows < 1 << 22
+    return (t.is_cuda and not _watched() and len(sh) == 4 and sh[3] == HEAD_DIM == buf.shape[-1] and sh[2] == rows < 1 << 22
             and sh[1] == buf.shape[1] and sh[0] < 512 and t.dtype == buf.dtype and t.dtype in _lib.DTYPES
             and t.get_device() == buf.get_device() and st[3] == 1 and not (st[0] | st[1] | st[2]) & 7
             and not t.data_ptr() & 15 and _plain(t) and _plain(buf))
@@ -117,7 +122,7 @@ def rows_ok(t, buf, rows):
 def _append_rows(kbuf, vbuf, row0, k, v):
     """Rows of the new tokens k/v to rows row0 .. of both buffers: one launch (tc_append_rows) for K and V where
     the kernel takes them, torch's two copies otherwise (host tensors, other types, head dims or broadcasts)."""
-    fast = _lib.FAST
+    fast = None if torch.compiler.is_compiling() else _lib.FAST
     if fast is not None and kbuf.is_cuda and fast.append_rows(kbuf, vbuf, row0, k, v,
                                                               _lib.raw_stream(kbuf.get_device())):
         return
