@@ -9,7 +9,7 @@ outputs' norm (1.6e-2 in bf16)."""
 import pytest
 import torch
 
-from threadcut_amd import paged, prefill, workloads
+from threadcut_amd import _lib, paged, prefill, workloads
 
 pytestmark = pytest.mark.gpu
 SCALE = 128 ** -0.5
@@ -177,3 +177,34 @@ def test_mask_map(gpu, ql, n, b, off, hq):
                 x, c = m[i, 0, rows, 64 * t:64 * t + 64].cpu(), causal[rows, 64 * t:64 * t + 64]
                 want = 0 if not x.any() else 1 if x.shape[1] == 64 and x.all() else 3 if torch.equal(x, c) else 2
                 assert got[i, blk, t] == want, (i, blk, t)
+
+
+@pytest.mark.parametrize("hq,hkv,ql,n", [(32, 8, 1, 1026), (32, 8, 3, 9000), (8, 2, 93, 4097), (32, 8, 100, 5000),
+                                         (16, 8, 200, 257)])
+def test_library_chosen_splits_need_the_workspace_the_query_tells(gpu, hq, hkv, ql, n):
+    """With num_splits 0 the call takes the splits of tc_prefill_num_splits, also for K/V whose rows lie too far
+    apart for one 32-bit range: the workspace of that count is enough, and all of it is needed."""
+    lib = _lib.load()
+    q, k, v = workloads.prefill_inputs(n, q_len=ql, n=n, q_heads=hq, kv_heads=hkv, device=gpu)
+    m, vis = masks("chunk", ql, n, 1, gpu, 0)
+    want = reference(q, k, v, vis, SCALE)
+    s = lib.tc_prefill_num_splits(1, ql, n, hq, hkv)
+    need = lib.tc_prefill_workspace_bytes(1, ql, hq, s)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=gpu)
+    stream = torch.cuda.current_stream().cuda_stream
+    wide = -(-2 ** 30 // (n + 128) // 8) * 8  # elements between tokens: just past 2^31 bytes for n + 128 rows
+    far = torch.zeros(2, n * wide, dtype=torch.float16, device=gpu).as_strided((2, hkv, n, 128), (n * wide, 128, wide, 1))
+    far[0], far[1] = k[0], v[0]
+    for kk, vv in ((k[0], v[0]), (far[0], far[1])):
+        for bytes_given in (need, need - 16):
+            out = torch.empty(1, ql, hq, 128, dtype=torch.float16, device=gpu)
+            rc = lib.tc_prefill_attention(
+                q.data_ptr(), _lib.i64x3(0, q.stride(1), q.stride(2)), kk.data_ptr(), _lib.i64x3(0, kk.stride(0), kk.stride(1)),
+                vv.data_ptr(), _lib.i64x3(0, vv.stride(0), vv.stride(1)), None, None, None, 0, 1, ql, n, 1, hq, hkv, 128,
+                _lib.TC_DTYPE_F16, SCALE, 0, ws.data_ptr(), max(bytes_given, 0), out.data_ptr(),
+                _lib.i64x3(0, hq * 128, 128), stream)
+            if bytes_given < need and s > 1:
+                assert rc == _lib.TC_ERR_WORKSPACE
+            else:
+                assert rc == _lib.TC_OK, lib.tc_last_error()
+                check(out, want, torch.float16)

@@ -1116,9 +1116,11 @@ struct Plan {
 //   - Tall where its splits leave less than 30% of the CUs idle: 93 on 9000: 29.8
 //     against 31.6 Wide, 31.0 Deep; 1024 on 9000: 169, 183; 300 on 9700: 65.8, 68.9.
 //   - else Wide: 600 on 7600 (W = 152): 99.7 in 3 splits against 114 Tall.
-// requested > 0 fixes the splits. Shapes other than Wide address a tile by one
-// 32-bit range over the slab (one_range); without it Wide takes the same splits.
-// Trailing empty splits are dropped: the result times its tiles covers n.
+// requested > 0 fixes the splits. Trailing empty splits are dropped: the result
+// times its tiles covers n. Shapes other than Wide address a tile by one 32-bit
+// range over the slab (one_range); without it Wide walks the very splits that
+// the call would have had, so that tc_prefill_num_splits, which does not know
+// the strides, tells the count of either.
 int plan(int batch, int64_t q_len, int64_t n, int group, int kv_heads, int requested, bool one_range, Plan* out) {
   int cus32 = 0;
   const int rc = current_device_cus(&cus32);
@@ -1147,13 +1149,17 @@ int plan(int batch, int64_t q_len, int64_t n, int group, int kv_heads, int reque
     shape = SHAPE_WIDE;
     s = fill(w, 2 * cus);
   }
-  if (!one_range) shape = SHAPE_WIDE;
-  const int64_t rows = shape == SHAPE_WIDE || shape == SHAPE_TALL ? 128 : 64;
+  const int64_t rows = shape == SHAPE_WIDE || shape == SHAPE_TALL || !one_range ? 128 : 64;
   const int64_t keys = shape == SHAPE_WIDE || shape == SHAPE_NARROW ? 64 : 128;
   if (requested > 0) s = std::min<int64_t>(requested, kMaxPrefillSplits);
   const int64_t ntiles = std::max<int64_t>(1, ceil_div(n, keys));
-  const int64_t st = ceil_div(ntiles, std::min(s, ntiles));
-  *out = Plan{shape, ceil_div(q_len, rows / group), st, static_cast<int>(ceil_div(ntiles, st))};
+  int64_t st = ceil_div(ntiles, std::min(s, ntiles));
+  const int64_t splits = ceil_div(ntiles, st);
+  if (!one_range) {
+    st *= keys / 64;
+    shape = SHAPE_WIDE;
+  }
+  *out = Plan{shape, ceil_div(q_len, rows / group), st, static_cast<int>(splits)};
   return TC_OK;
 }
 
