@@ -145,6 +145,11 @@ def test_prefill_validation_before_any_device_call(lib):
     assert prefill(hq=24) == _lib.TC_ERR_UNSUPPORTED                   # group 3
     assert prefill(q_len=65) == _lib.TC_ERR_INVALID_ARGUMENT           # more queries than keys
     assert prefill(q=4100) == _lib.TC_ERR_ALIGNMENT
+    # Up to 2^27 query blocks of all heads and sequences pass the check of the grid (and then, here, meet another one).
+    many = lambda hkv: lib.tc_prefill_attention(4096, st, 8192, st, 12288, st, None, None, 16384, 0, 1, 1, 1, 65535, hkv,
+                                                hkv, 128, 0, 0.088, 0, None, 0, 16384, st, None)
+    assert many(2047) == _lib.TC_ERR_INVALID_ARGUMENT and b"without its mask" in lib.tc_last_error()
+    assert many(2049) == _lib.TC_ERR_UNSUPPORTED and b"grid" in lib.tc_last_error()
     # Key positions are 32-bit in the kernel: 2^30 keys or more are refused.
     assert prefill(n=1 << 30) == _lib.TC_ERR_UNSUPPORTED
     assert b"2^30" in lib.tc_last_error()

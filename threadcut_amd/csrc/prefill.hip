@@ -1273,7 +1273,8 @@ int prefill_impl(const void* q_dev, const int64_t q_strides[3], const void* k_de
   if (!std::isfinite(scale)) return fail(TC_ERR_INVALID_ARGUMENT, "scale is not finite");
   int64_t nblk, ntiles;
   tile_geometry(q_len, n_tokens, group, &nblk, &ntiles);
-  if (2 * nblk * kv_heads * batch * kMaxPrefillSplits > 0x7fffffff) return fail(TC_ERR_UNSUPPORTED, "grid too large");
+  // 2^27 query blocks; the grid that the splits make of them is checked with the plan.
+  if (nblk * kv_heads * batch * 16 > 0x7fffffff) return fail(TC_ERR_UNSUPPORTED, "grid too large");
   if (mask_dev) {
     if (causal) return fail(TC_ERR_INVALID_ARGUMENT, "pass either a mask or causal, not both");
     if ((rc = check_mask_strides(mask_strides)) != TC_OK) return rc;
@@ -1293,6 +1294,7 @@ int prefill_impl(const void* q_dev, const int64_t q_strides[3], const void* k_de
   Plan p;
   if ((rc = plan(batch, q_len, n_tokens, group, kv_heads, num_splits, pools || whole, &p)) != TC_OK) return rc;
   const int splits = p.splits;
+  if (p.nblk * kv_heads * batch * splits > 0x7fffffff) return fail(TC_ERR_UNSUPPORTED, "grid too large");
   const size_t need = workspace_bytes(batch, q_len, q_heads, splits);
   if (need > 0 && (!workspace_dev || workspace_bytes_in < need))
     return fail(TC_ERR_WORKSPACE, "%d key splits need %zu workspace bytes, got %zu", splits, need,
