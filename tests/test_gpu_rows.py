@@ -181,6 +181,20 @@ def test_append_is_recorded_by_tracing(gpu, monkeypatch, kind):
         assert torch.equal(torch.compile(g, backend="eager", fullgraph=True)(b), torch.cat((a, b), 2))
 
 
+@pytest.mark.parametrize("native", [True, False])
+def test_append_of_more_rows_than_the_kernel_takes(gpu, monkeypatch, native):
+    """65535 tiles of 64 rows fill the kernel's grid; one row more goes through torch."""
+    if not native:
+        _lib.load()
+        monkeypatch.setattr(_lib, "FAST", None)
+    for n in (64 * 65535, 64 * 65535 + 1):
+        layer = kv.GrowingLayer()
+        k, v = (rows("heads first", 1, 1, 1, torch.float16, gpu, i).expand(1, 1, n, 128) for i in (1, 2))
+        layer.update(k, v)
+        assert kv.rows_ok(k, layer.kbuf, n) == (n == 64 * 65535)
+        assert torch.equal(layer.kbuf, k) and torch.equal(layer.vbuf, v)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("form", [f for f in KERNEL + TORCH if f != "broadcast batch"])
 @pytest.mark.parametrize("layers,P,n", [(1, 16, 1), (3, 64, 65), (70, 16, 37)])

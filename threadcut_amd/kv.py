@@ -25,6 +25,7 @@ from .flash_decode import _on_device
 from .match import Split  # noqa: F401  (re-exported: the splice contract)
 
 HEAD_DIM = 128
+MAX_ROWS = 64 * 65535  # new tokens per launch of the row-writing kernels (tiles of 64 in the grid's second dimension)
 
 # Deferred single-token appends of GrowingLayers in fused-append mode, by the
 # address of the layer's K buffer; the "threadcut" attention takes them.
@@ -113,7 +114,7 @@ def rows_ok(t, buf, rows):
     with strides of whole 16-byte chunks, within the launch grid, and a buffer that autograd does not track. Whoever
     launches such a kernel tells autograd of the write (increment_version), as torch's copy would."""
     sh, st = t.shape, t.stride()
-    return (t.is_cuda and not _watched() and len(sh) == 4 and sh[3] == HEAD_DIM == buf.shape[-1] and sh[2] == rows < 1 << 22
+    return (t.is_cuda and not _watched() and len(sh) == 4 and sh[3] == HEAD_DIM == buf.shape[-1] and sh[2] == rows <= MAX_ROWS
             and sh[1] == buf.shape[1] and sh[0] < 512 and t.dtype == buf.dtype and t.dtype in _lib.DTYPES
             and t.get_device() == buf.get_device() and st[3] == 1 and not (st[0] | st[1] | st[2]) & 7
             and not t.data_ptr() & 15 and _plain(t) and _plain(buf))
