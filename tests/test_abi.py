@@ -1,11 +1,16 @@
 """The C ABI without a GPU: the library loads, exports every symbol the header
 declares, and rejects bad arguments before it touches the device."""
 import ctypes
+import importlib.util
 import os
 import re
+import sys
+import types
 
 import pytest
+import torch
 
+import threadcut_amd
 from threadcut_amd import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -212,6 +217,34 @@ def test_append_validation(lib):
     assert paged(pages=0) == _lib.TC_ERR_INVALID_ARGUMENT
     assert paged(k=_lib.ptr_array([0])) == _lib.TC_ERR_INVALID_ARGUMENT
     assert paged(layers=0, slots=None) == _lib.TC_OK
+
+
+@pytest.mark.parametrize("fault", ["absent", "another torch"])
+def test_missing_native_paths_leave_the_python_ones(monkeypatch, fault):
+    """The library loads without _fast.so, or with one built against another torch: a warning, and no native paths."""
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "FAST", None)
+    fake = None  # (None in sys.modules: the import fails)
+    if fault == "another torch":
+        fake = types.ModuleType("threadcut_amd._fast")
+        fake.torch_version = "0.0"
+    monkeypatch.setitem(sys.modules, "threadcut_amd._fast", fake)
+    monkeypatch.delattr(threadcut_amd, "_fast", raising=False)
+    if fake:
+        monkeypatch.setattr(threadcut_amd, "_fast", fake, raising=False)
+    with pytest.warns(RuntimeWarning, match="native call paths"):
+        assert _lib.load().tc_abi_version() == 2
+    assert _lib.FAST is None
+
+
+def test_import_on_a_torch_without_the_raw_stream_getter(monkeypatch):
+    """The package imports (its CPU path needs no GPU build of torch) and takes the stream from the Stream object."""
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    spec = importlib.util.spec_from_file_location("threadcut_amd._lib_copy", _lib.__file__)
+    copy = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(copy)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda index: types.SimpleNamespace(cuda_stream=7 + index))
+    assert copy.raw_stream(3) == 10
 
 
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):

@@ -9,6 +9,7 @@ import ctypes
 import functools
 import os
 import threading
+import warnings
 
 import torch
 
@@ -92,7 +93,7 @@ SIGNATURES = {
 _lock = threading.Lock()
 _lib = None
 # The native call paths (csrc/host/fastcall.cpp, linked against the default library): None until the library is
-# loaded, and while `using` has another build in its place.
+# loaded, where they do not load, and while `using` has another build in its place.
 FAST = None
 
 
@@ -112,13 +113,22 @@ def load():
                 fn = getattr(lib, name)
                 fn.restype = res
                 fn.argtypes = args
-            try:
-                from . import _fast
-            except ImportError as e:
-                raise RuntimeError(f"threadcut_amd: the native call paths (_fast.so) do not load ({e}); build them "
-                                   "with `python -m threadcut_amd.build`.") from e
-            _lib, FAST = lib, _fast
+            _lib, FAST = lib, _native_paths()
     return _lib
+
+
+def _native_paths():
+    """The _fast module, or None (with a warning) where it does not load or was built against another torch, whose
+    tensors it could misread: every call then takes its Python path to the same kernels."""
+    try:
+        from . import _fast
+        if _fast.torch_version != torch.__version__:
+            raise ImportError(f"built against torch {_fast.torch_version}, this is {torch.__version__}")
+    except ImportError as e:
+        warnings.warn(f"threadcut_amd: the native call paths (_fast.so) are left out ({e}); calls cost more host time. "
+                      "Build them with `python -m threadcut_amd.build`.", RuntimeWarning, stacklevel=3)
+        return None
+    return _fast
 
 
 def bind(path):
@@ -187,7 +197,12 @@ def float_array(t):
     return (ctypes.c_float * t.numel())(*t.tolist())
 
 
-raw_stream = torch._C._cuda_getCurrentRawStream  # the current stream of a device index, as a whole number
+def _raw_stream(index):
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+# The current stream of a device index, as a whole number (torch's own getter where this build of torch has it).
+raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _raw_stream)
 
 
 def stream_of(device):

@@ -80,7 +80,7 @@ def _compile_fast(obj):
 
     system = [x for p in (*include_paths(), sysconfig.get_paths()["include"]) for x in ("-isystem", p)]
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           *system, "-c", os.path.join(CSRC, "host", "fastcall.cpp"), "-o", obj]
+           f'-DTC_TORCH_VERSION="{torch.__version__}"', *system, "-c", os.path.join(CSRC, "host", "fastcall.cpp"), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"g++ failed on fastcall.cpp:\n{r.stderr}")

@@ -307,5 +307,8 @@ PyMODINIT_FUNC PyInit__fast() {
       {"append_rows", fast(append_rows), METH_FASTCALL, "append_rows(k_buf, v_buf, row0, k, v, stream) -> bool"},
       {nullptr, nullptr, 0, nullptr}};
   static PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fast", "Native call paths of the wrappers.", -1, methods};
-  return PyModule_Create(&module);
+  PyObject* m = PyModule_Create(&module);
+  // The torch whose headers these paths were compiled with: they read its tensors in place, so they serve no other.
+  if (m && PyModule_AddStringConstant(m, "torch_version", TC_TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
 }
