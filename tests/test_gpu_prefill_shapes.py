@@ -75,6 +75,20 @@ def test_shapes(gpu, hq, hkv, ql, n, mode):
     check(out, reference(q, k, v, vis, SCALE), dtype)
 
 
+@pytest.mark.parametrize("mode", ["causal", "padded"])
+@pytest.mark.parametrize("hq,hkv,ql,n,b", [(8, 2, 300, 300, 5), (32, 8, 700, 900, 3), (64, 16, 290, 290, 9),
+                                           (16, 16, 150, 1100, 7), (32, 32, 130, 650, 6)])
+def test_batches(gpu, hq, hkv, ql, n, b, mode):
+    """Several sequences, in both orders of their blocks: prompts of few and of many rounds, and chunks."""
+    if mode == "causal" and 2 * ql < n:
+        mode = "chunk"
+    q, k, v = workloads.prefill_inputs(ql + b, batch=b, q_len=ql, n=n, q_heads=hq, kv_heads=hkv, dtype=torch.float16,
+                                       device=gpu)
+    m, vis = masks(mode, ql, n, b, gpu, n)
+    out = prefill.prefill_attention(q, k, v, m, SCALE, mode == "causal")
+    check(out, reference(q, k, v, vis, SCALE), torch.float16)
+
+
 @pytest.mark.parametrize("splits", [2, 3, 5, 9, 17, 32, 40])
 @pytest.mark.parametrize("hq,hkv,ql,n", [(32, 8, 5, 3000), (32, 8, 100, 5000), (16, 8, 200, 257), (32, 8, 600, 5001)])
 def test_split_counts(gpu, hq, hkv, ql, n, splits):
