@@ -55,7 +55,9 @@ def check(out, want, dtype):
 # (q_heads, kv_heads, queries, keys): which shape 256 compute units give, at and around its tiles' edges.
 SIZES = [
     (32, 8, 1, 1), (32, 8, 17, 33), (8, 2, 64, 64), (16, 8, 200, 257), (64, 8, 300, 639),    # 64 rows, two key groups
+    (32, 8, 14, 43), (8, 8, 1, 64), (16, 2, 9, 65), (32, 4, 31, 320),                        # (chunks on a few keys)
     (16, 8, 700, 700), (8, 8, 127, 641), (32, 8, 5, 3000), (8, 2, 93, 4097), (64, 8, 8, 2111),  # 64 rows, four
+    (32, 4, 31, 321),
     (32, 8, 1100, 1100), (32, 8, 100, 5000), (64, 8, 129, 4223), (8, 8, 1500, 7000),         # 128 rows, two
     (64, 8, 1030, 1030), (32, 8, 600, 5001),                                                 # 128 rows, one
 ]

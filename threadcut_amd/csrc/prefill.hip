@@ -1114,6 +1114,9 @@ struct Plan {
 //     Deep; 2048: 46.6, 51.2, 65.4.
 // - A chunk on a longer cache is split to fill the CUs once (a second round
 //   would double the call), into at most 32 splits of at least 256 keys.
+//   - T <= 5: Narrow, Wide where W64 > C. A Deep tile of 128 keys is mostly empty
+//     there: 14 tokens on 43 of 32 heads 6.5 us against 7.8 Deep, 6.3 Wide; at T = 2
+//     0.83 of Deep's time over 366 shapes, 0.97 at 5, 1.02 at 6 and 7.
 //   - Deep for few rows (W64 <= C / 6) or short caches (n <= 4096, W64 <= 7/8 C):
 //     3 tokens on 9000: 15.6 against 17.3 Wide, 16.9 Tall; 150 on 1500: 19.7,
 //     22.3, 22.2; 400 on 3000: 38.1, 43.0, 41.7.
@@ -1143,6 +1146,8 @@ int plan(int batch, int64_t q_len, int64_t n, int group, int kv_heads, int reque
       shape = SHAPE_DEEP;
     else
       shape = w > 2 * cus || (w > cus && T <= 16) ? SHAPE_WIDE : SHAPE_TALL;
+  } else if (T <= 5) {
+    shape = w64 <= cus ? SHAPE_NARROW : SHAPE_WIDE;
   } else if (6 * w64 <= cus || (n <= 4096 && 8 * w64 <= 7 * cus)) {
     shape = SHAPE_DEEP;
     s = fill(w64, cus);
