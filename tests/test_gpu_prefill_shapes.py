@@ -59,6 +59,7 @@ SIZES = [
     (16, 8, 700, 700), (8, 8, 127, 641), (32, 8, 5, 3000), (8, 2, 93, 4097), (64, 8, 8, 2111),  # 64 rows, four
     (32, 4, 31, 321),
     (32, 8, 1100, 1100), (32, 8, 100, 5000), (64, 8, 129, 4223), (8, 8, 1500, 7000),         # 128 rows, two
+    (16, 8, 1300, 1300),                                                                     # (W64 = 1.3 C, W < C)
     (64, 8, 1030, 1030), (32, 8, 600, 5001),                                                 # 128 rows, one
 ]
 

@@ -1105,6 +1105,10 @@ struct Plan {
 //   work-groups: the combine costs more than it saves.
 //   - T <= 10, W <= C: Narrow (64 rows, two key groups). 300 tokens 10.1 against
 //     11.8 Wide, 10.7 Deep; four prompts of 300 (W > C): Wide, 13.6 against 16.4.
+//   - No mask and not causal, so that every block walks all tiles: a work-group more
+//     than the CUs costs a round. Deep for W64 <= C, Tall for W <= C, else Wide. 656
+//     of 32 heads (W64 = 328): 18.1 Tall, 27.3 Deep, 20.0 Wide; 1329 of 32 over 8 (W
+//     = 336): 48 Wide, 52 Tall.
 //   - W64 <= 4/3 C: Deep, a quarter of the tiles in a row. 1100 tokens of 16
 //     heads over 8: 18.3 against 26.8 Wide, 22.4 Tall; 1300: 21.5, 30.5, 24.2.
 //   - W > 2 C, or W > C with few tiles: Wide, two independent work-groups a CU.
@@ -1128,7 +1132,9 @@ struct Plan {
 // range over the slab (one_range); without it Wide walks the very splits that
 // the call would have had, so that tc_prefill_num_splits, which does not know
 // the strides, tells the count of either.
-int plan(int batch, int64_t q_len, int64_t n, int group, int kv_heads, int requested, bool one_range, Plan* out) {
+// even: every query sees every key (the splits do not depend on it).
+int plan(int batch, int64_t q_len, int64_t n, int group, int kv_heads, int requested, bool one_range, bool even,
+         Plan* out) {
   int cus32 = 0;
   const int rc = current_device_cus(&cus32);
   if (rc != TC_OK) return rc;
@@ -1142,6 +1148,8 @@ int plan(int batch, int64_t q_len, int64_t n, int group, int kv_heads, int reque
   if (2 * q_len >= n) {
     if (T <= 10)
       shape = w <= cus ? SHAPE_NARROW : SHAPE_WIDE;
+    else if (even)
+      shape = w64 <= cus ? SHAPE_DEEP : w <= cus ? SHAPE_TALL : SHAPE_WIDE;
     else if (3 * w64 <= 4 * cus)
       shape = SHAPE_DEEP;
     else
@@ -1188,7 +1196,7 @@ extern "C" int tc_prefill_num_splits(int batch, int64_t q_len, int64_t n_tokens,
   if (batch < 1 || q_len < 0 || n_tokens < q_len) return -fail(TC_ERR_INVALID_ARGUMENT, "batch %d, q_len %lld, n %lld", batch, (long long)q_len, (long long)n_tokens);
   if ((rc = check_group(q_heads, kv_heads, &group)) != TC_OK) return -rc;
   Plan p;
-  if ((rc = plan(batch, q_len, n_tokens, group, kv_heads, 0, true, &p)) != TC_OK) return -rc;
+  if ((rc = plan(batch, q_len, n_tokens, group, kv_heads, 0, true, false, &p)) != TC_OK) return -rc;
   return p.splits;
 }
 
@@ -1301,7 +1309,8 @@ int prefill_impl(const void* q_dev, const int64_t q_strides[3], const void* k_de
   // One 32-bit buffer range over a head's slab, with room for the tiles' rows past n.
   const bool whole = !pools && (n_tokens + 2 * kKeys) * 2 * std::max(k_strides[2], v_strides[2]) < (int64_t(1) << 31);
   Plan p;
-  if ((rc = plan(batch, q_len, n_tokens, group, kv_heads, num_splits, pools || whole, &p)) != TC_OK) return rc;
+  if ((rc = plan(batch, q_len, n_tokens, group, kv_heads, num_splits, pools || whole, !causal && !mask_dev,
+                 &p)) != TC_OK) return rc;
   const int splits = p.splits;
   if (p.nblk * kv_heads * batch * splits > 0x7fffffff) return fail(TC_ERR_UNSUPPORTED, "grid too large");
   const size_t need = workspace_bytes(batch, q_len, q_heads, splits);
