@@ -1121,11 +1121,15 @@ struct Plan {
 //   - T <= 5: Narrow, Wide where W64 > C. A Deep tile of 128 keys is mostly empty
 //     there: 14 tokens on 43 of 32 heads 6.5 us against 7.8 Deep, 6.3 Wide; at T = 2
 //     0.83 of Deep's time over 366 shapes, 0.97 at 5, 1.02 at 6 and 7.
-//   - Deep for few rows (W64 <= C / 6) or short caches (n <= 4096, W64 <= 7/8 C):
+//   - Deep for few rows (W64 <= C / 6) or short caches (n <= 4096 and two splits, W64
+//     <= C / 2; n <= 3072, W64 <= 7/8 C: 0.82 of Wide's time with T in [16, 24), 1.03
+//     in [56, 64)):
 //     3 tokens on 9000: 15.6 against 17.3 Wide, 16.9 Tall; 150 on 1500: 19.7,
 //     22.3, 22.2; 400 on 3000: 38.1, 43.0, 41.7.
-//   - Tall where its splits leave less than 30% of the CUs idle: 93 on 9000: 29.8
-//     against 31.6 Wide, 31.0 Deep; 1024 on 9000: 169, 183; 300 on 9700: 65.8, 68.9.
+//   - Tall where its splits fill at least 0.85 as much of the CUs as Wide's fill of
+//     their two slots: 93 on 9000: 29.8 against 31.6 Wide, 31.0 Deep; 1024 on 9000:
+//     169, 183; 300 on 9700: 65.8, 68.9. With W = 96 (2 splits Tall, 5 Wide): 189 on
+//     16238 142 Tall, 132 Wide.
 //   - else Wide: 600 on 7600 (W = 152): 99.7 in 3 splits against 114 Tall.
 // requested > 0 fixes the splits. Trailing empty splits are dropped: the result
 // times its tiles covers n. Shapes other than Wide address a tile by one 32-bit
@@ -1156,10 +1160,10 @@ int plan(int batch, int64_t q_len, int64_t n, int group, int kv_heads, int reque
       shape = w > 2 * cus || (w > cus && T <= 16) ? SHAPE_WIDE : SHAPE_TALL;
   } else if (T <= 5) {
     shape = w64 <= cus ? SHAPE_NARROW : SHAPE_WIDE;
-  } else if (6 * w64 <= cus || (n <= 4096 && 8 * w64 <= 7 * cus)) {
+  } else if (6 * w64 <= cus || (n <= 4096 && 2 * w64 <= cus) || (n <= 3072 && 8 * w64 <= 7 * cus)) {
     shape = SHAPE_DEEP;
     s = fill(w64, cus);
-  } else if (w <= cus && 10 * w * fill(w, cus) >= 7 * cus) {
+  } else if (w <= cus && 40 * fill(w, cus) >= 17 * fill(w, 2 * cus)) {
     shape = SHAPE_TALL;
     s = fill(w, cus);
   } else {
