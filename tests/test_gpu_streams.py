@@ -155,9 +155,9 @@ def zeros_to_reuse(shape, dtype, gpu):
     torch.zeros(shape, dtype=dtype, device=gpu)
 
 
-def test_a_mask_map_is_waited_for_by_other_streams(gpu):
+def test_a_mask_map_on_other_streams(gpu):
     """The tile map of a mask is built on the stream of its first call; a call on another stream that meets the same
-    mask waits for it."""
+    mask does not read it before it is there."""
     b, hq, hkv, ql, n = 1, 32, 8, 200, 900
     q, k, v = (rnd(s, i).to(gpu) for i, s in enumerate(((b, hq, ql, D), (b, hkv, n, D), (b, hkv, n, D))))
     m = (torch.arange(n, device=gpu)[None, :] <= torch.arange(ql, device=gpu)[:, None] + (n - ql))[None, None]
@@ -185,9 +185,9 @@ class TwoLayers:
         return self
 
 
-def test_paged_slots_are_waited_for_by_other_streams(gpu):
+def test_paged_slots_on_other_streams(gpu):
     """The slot list of a chunk is uploaded by the first layer's append; another layer's append on another stream
-    waits for it."""
+    does not read it before it is there."""
     n = 40
     k = [rnd((1, 8, n, D), i).to(gpu) for i in range(2)]
     cache = new_paged_cache(TwoLayers(), 8, 16)
@@ -209,9 +209,9 @@ def test_paged_slots_are_waited_for_by_other_streams(gpu):
         assert torch.equal(gk, want) and torch.equal(gv, want)
 
 
-def test_paged_tables_are_waited_for_by_other_streams(gpu):
+def test_paged_tables_on_other_streams(gpu):
     """The tile table and the token offsets are uploaded by the first call that reads them; decode and prefill calls
-    on another stream wait for them."""
+    on another stream do not read them before they are there."""
     n = 300
     k, q, qp = rnd((8, n, D), 1).to(gpu), rnd((1, 8, 4, D), 2).to(gpu), rnd((1, 32, 20, D), 3).to(gpu)
     want = None

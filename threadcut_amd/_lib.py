@@ -212,26 +212,18 @@ def stream_of(device):
     return ctypes.c_void_p(raw_stream(torch.cuda.current_device() if index is None else index))
 
 
-class Resident:
-    """Device tensors that one call makes and later calls read, on its stream or on others. A reader on another stream
-    knows nothing of the work that made them, so ``get`` makes its stream wait for that work, and keeps the memory
-    until the reads are done. (Not under graph capture, where a wait for uncaptured work is refused: what a capture
-    reads has to be finished before it begins.)"""
-
-    def __init__(self, *tensors):
-        self.tensors = tensors
-        self.index = tensors[0].get_device()
-        self.stream = raw_stream(self.index)
-        self.made = torch.cuda.Event()
-        self.made.record(torch.cuda.current_stream(self.index))
-
-    def get(self):
-        if raw_stream(self.index) != self.stream and not torch.cuda.is_current_stream_capturing():
-            here = torch.cuda.current_stream(self.index)
-            here.wait_event(self.made)
-            for t in self.tensors:
-                t.record_stream(here)
-        return self.tensors
+def per_stream(copies, index, make):
+    """What `make` returns (device tensors that later calls read), one copy for every stream of GPU `index` that asks,
+    kept in the dict `copies`. A reader on another stream knows nothing of the work that made a copy and would have to
+    wait for it, and keep its memory until the read is done; an event for that costs each new copy 10 us. Under graph
+    capture any copy serves: an upload cannot be captured, and what a capture reads has to be finished before it begins."""
+    stream = raw_stream(index)
+    hit = copies.get(stream)
+    if hit is None:
+        if copies and torch.cuda.is_current_stream_capturing():
+            return next(iter(copies.values()))
+        hit = copies[stream] = make()
+    return hit
 
 
 def require_gpu(*tensors, what):

@@ -94,7 +94,7 @@ def _splice_layer_torch(kbuf, vbuf, s, inv_freq):
         vbuf[..., s.a:s.a + s.c, :] = v
 
 
-def _watched():
+def watched():
     """True while torch records every operation: compilation, torch.jit.trace, a dispatch mode (make_fx), a functorch
     transform, forward mode. Writes stay torch ops then."""
     return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0
@@ -112,9 +112,10 @@ def rows_ok(t, buf, rows):
     """True if the row-writing kernels take `t` as `rows` new tokens of the cache buffer or pool `buf`
     ([*, heads, *, 128]): a plain [batch, heads, rows, 128] view in the buffer's type and device, 16-byte aligned
     with strides of whole 16-byte chunks, within the launch grid, and a buffer that autograd does not track. Whoever
-    launches such a kernel tells autograd of the write (increment_version), as torch's copy would."""
+    launches such a kernel asks `watched` first, and tells autograd of the write (increment_version), as torch's copy
+    would."""
     sh, st = t.shape, t.stride()
-    return (t.is_cuda and not _watched() and len(sh) == 4 and sh[3] == HEAD_DIM == buf.shape[-1] and sh[2] == rows <= MAX_ROWS
+    return (t.is_cuda and len(sh) == 4 and sh[3] == HEAD_DIM == buf.shape[-1] and sh[2] == rows <= MAX_ROWS
             and sh[1] == buf.shape[1] and sh[0] < 512 and t.dtype == buf.dtype and t.dtype in _lib.DTYPES
             and t.get_device() == buf.get_device() and st[3] == 1 and not (st[0] | st[1] | st[2]) & 7
             and not t.data_ptr() & 15 and _plain(t) and _plain(buf))
@@ -129,7 +130,7 @@ def _append_rows(kbuf, vbuf, row0, k, v):
         return
     add, sb = k.shape[-2], kbuf.stride()
     if (k.is_cuda and add and len(sb) == 4 and kbuf.shape[0] == k.shape[0] and k.shape == v.shape
-            and sb == vbuf.stride() and rows_ok(k, kbuf, add) and rows_ok(v, vbuf, add)):
+            and sb == vbuf.stride() and not watched() and rows_ok(k, kbuf, add) and rows_ok(v, vbuf, add)):
         b, h, cap, d = kbuf.shape
         sk, sv = k.stride(), v.stride()
         with _on_device(kbuf.device):

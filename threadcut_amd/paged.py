@@ -38,7 +38,7 @@ from transformers.cache_utils import DynamicLayer
 
 from . import _lib
 from .flash_decode import HEAD_DIM, _on_device, _plan
-from .kv import rope_table, rows_ok
+from .kv import rope_table, rows_ok, watched
 from .prefill import GROUPS
 
 TILE = 16  # rows per tile-table entry (the decode kernel's tile)
@@ -253,7 +253,8 @@ class PagedKV:
         # The pools' own device, with its index ("cuda" alone names the current device).
         self.device = self.k_pools[0].device if self.k_pools else torch.device(
             "cuda", torch.cuda.current_device() if dev.index is None else dev.index)
-        self._dev_table = None  # (version, (table, tiles) on the device, max_tiles)
+        # (version, what device_table or device_offsets returns, for each stream)
+        self._dev_table = self._dev_off = (None, None)
 
     @property
     def layers(self):
@@ -292,6 +293,8 @@ class PagedKV:
         """New tokens' rows, per layer [B, Hkv, n, D], into the pools' slots (int64 [B, n, 2] of (page, slot) on the
         device, or [n, 2] for one sequence) with one launch (tc_paged_append_rows). False if the kernel does not
         take the tensors (another type, strides that differ between layers): nothing is written then."""
+        if watched():
+            return False
         b, n = (1, slots.shape[0]) if slots.dim() == 2 else slots.shape[:2]
         k0, v0 = ks[0], vs[0]
         for i, k, v in zip(layers, ks, vs):
@@ -324,25 +327,32 @@ class PagedKV:
 
     def device_table(self):
         """(tile table int32 [B, max_tiles, 4], tiles int32 [B], max_tiles) on the device."""
-        ver = self.table.version
-        if self._dev_table is None or self._dev_table[0] != ver:
-            tab, cnt = self.table.tile_table()
-            self._dev_table = (ver, _lib.Resident(_to_device(tab, self.device), _to_device(cnt, self.device)),
-                               tab.shape[1])
-        _, tables, max_tiles = self._dev_table
-        return (*tables.get(), max_tiles)
+        version, copies = self._dev_table
+        if version != self.table.version:
+            copies = {}
+            self._dev_table = (self.table.version, copies)
+        return (copies.get(_lib.raw_stream(self.device.index))
+                or _lib.per_stream(copies, self.device.index, self._upload_table))
+
+    def _upload_table(self):
+        tab, cnt = self.table.tile_table()
+        return _to_device(tab, self.device), _to_device(cnt, self.device), tab.shape[1]
 
     def device_offsets(self):
         """(token offsets int32 [B, pitch], pitch) on the device: the byte offset of each logical
         token's row in a head slab of the pools (PageTable.token_offsets), for the paged prefill
         and the device-length decode step."""
-        ver = self.table.version
-        if getattr(self, "_dev_off", None) is None or self._dev_off[0] != ver:
-            st = self.k_pools[0].stride()
-            off = self.table.token_offsets(st[0] * 2, st[2] * 2)
-            self._dev_off = (ver, _lib.Resident(_to_device(off, self.device)), off.shape[1])
-        _, offsets, pitch = self._dev_off
-        return (*offsets.get(), pitch)
+        version, copies = self._dev_off
+        if version != self.table.version:
+            copies = {}
+            self._dev_off = (self.table.version, copies)
+        return (copies.get(_lib.raw_stream(self.device.index))
+                or _lib.per_stream(copies, self.device.index, self._upload_offsets))
+
+    def _upload_offsets(self):
+        st = self.k_pools[0].stride()
+        off = self.table.token_offsets(st[0] * 2, st[2] * 2)
+        return _to_device(off, self.device), off.shape[1]
 
     def prefill(self, layer, query, scale, mask=None, causal=False, out=None):
         """The prefill branch of threadcut/attention.py:43-46 over the pools: query
@@ -661,15 +671,12 @@ class PagedCacheState:
 
     def slots_on_device(self, lo, hi):
         """(page, slot) of every sequence's positions [lo, hi), int64 [B, hi - lo, 2] on the device; every
-        layer of a step writes the same positions, so the upload is kept for the table version."""
+        layer of a step writes the same positions, so the upload is kept (for each stream) for the table version."""
         key = (self.kv.table.version, lo, hi)
-        hit = self._slots.get(key)
-        if hit is None:
-            if self._slots and next(iter(self._slots))[0] != key[0]:
-                self._slots.clear()
-            slots = np.stack([self.kv.table.token_slots(b)[lo:hi] for b in range(self.batch)])
-            hit = self._slots[key] = _lib.Resident(_to_device(slots, self.kv.device))
-        return hit.get()[0]
+        if self._slots and next(iter(self._slots))[0] != key[0]:
+            self._slots.clear()
+        return _lib.per_stream(self._slots.setdefault(key, {}), self.kv.device.index, lambda: _to_device(
+            np.stack([self.kv.table.token_slots(b)[lo:hi] for b in range(self.batch)]), self.kv.device))
 
     def reserve_step_for(self, layer):
         """A decode step's slot per sequence: reserved by the first layer of the step."""

@@ -118,7 +118,7 @@ def prefill_attention(query, key, value, attention_mask=None, scale=None, is_cau
     return out
 
 
-# The tile map of the last mask seen. transformers builds one mask per forward
+# The tile map of the last mask seen, for each stream. transformers builds one mask per forward
 # pass and hands the same tensor to every layer, so the map is built once per
 # pass; it is rebuilt when the mask object, its version or the geometry change.
 # A captured call builds its own: a replay must not read a map that it did not
@@ -129,10 +129,20 @@ _tile_cache = None
 def mask_tiles(mask, q_heads, kv_heads):
     """uint8 tile map of a bool mask [b|1, 1, q, n] (``tc_prefill_mask_tiles``), cached per mask."""
     global _tile_cache
-    key = (mask._version, tuple(mask.shape), tuple(mask.stride()), mask.data_ptr(), q_heads, kv_heads)
-    c, captured = _tile_cache, torch.cuda.is_current_stream_capturing()
-    if c is not None and not captured and c[0]() is mask and c[1] == key:
-        return c[2].get()[0]
+    if torch.cuda.is_current_stream_capturing():
+        return _build_tiles(mask, q_heads, kv_heads)
+    key = (mask._version, mask.shape, mask.stride(), mask.data_ptr(), q_heads, kv_heads)
+    c = _tile_cache
+    if c is None or c[0]() is not mask or c[1] != key:
+        c = _tile_cache = (weakref.ref(mask), key, {})
+    index = mask.get_device()
+    tiles = c[2].get(_lib.raw_stream(index))
+    if tiles is None:
+        tiles = _lib.per_stream(c[2], index, lambda: _build_tiles(mask, q_heads, kv_heads))
+    return tiles
+
+
+def _build_tiles(mask, q_heads, kv_heads):
     m = mask[:, 0]
     mb = m.shape[0] if m.shape[0] > 1 and m.stride(0) != 0 else 1
     q, n = m.shape[1], m.shape[2]
@@ -144,6 +154,4 @@ def mask_tiles(mask, q_heads, kv_heads):
         rc = lib.tc_prefill_mask_tiles(m.data_ptr(), st, mb, q, n, q_heads, kv_heads, tiles.data_ptr(),
                                        tiles.numel(), _lib.stream_of(mask.device))
     _lib.check(rc, "tc_prefill_mask_tiles")
-    if not captured:
-        _tile_cache = (weakref.ref(mask), key, _lib.Resident(tiles))
     return tiles
