@@ -806,6 +806,13 @@ __global__ __launch_bounds__(64 * S::kWaves) __attribute__((amdgpu_waves_per_eu(
     uint16_t* p = at < kBuf ? s_k0 : at < 2 * kBuf ? s_k1 : at < 3 * kBuf ? s_v0 : s_v1;
     stage = reinterpret_cast<char*>(p) + at % kBuf;
   }
+  // The lanes of a wave read rows that other lanes of it have written: its LDS
+  // accesses run in order, and this keeps the compiler to that order.
+  auto staged = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
   const int d0 = kOwnDims * kg;  // the wave's first dim
   const bool partial = a.splits > 1;
   const int64_t prow0 = ((static_cast<int64_t>(b) * splits + split) * a.q_len) * (a.kv_heads * G);
@@ -824,6 +831,7 @@ __global__ __launch_bounds__(64 * S::kWaves) __attribute__((amdgpu_waves_per_eu(
           *reinterpret_cast<uint2*>(stage + r32 * (16 * kC) + 16 * (c ^ (r32 & (kC - 1))) + 8 * hi) = make_uint2(w0, w1);
         }
       }
+    staged();
     uint16_t* const ob = a.out + b * a.so_b + static_cast<int64_t>(h) * G * a.so_h + d0;
 #pragma unroll
     for (int i = 0; i < kC / 2; ++i) {
@@ -844,6 +852,7 @@ __global__ __launch_bounds__(64 * S::kWaves) __attribute__((amdgpu_waves_per_eu(
               o[dt][4 * j] * inv, o[dt][4 * j + 1] * inv, o[dt][4 * j + 2] * inv, o[dt][4 * j + 3] * inv);
         }
       }
+    staged();
     float* const ob = a.o_part + prow0 * kHeadDim + d0;
 #pragma unroll
     for (int i = 0; i < kC / 2; ++i) {
