@@ -398,7 +398,7 @@ def test_interleaved_partials_cover_round_robin_tiles(gpu, n, split):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("b,hkv,g,n", [(1, 8, 4, 1), (1, 8, 1, 64), (3, 2, 8, 63), (32, 8, 4, 300), (64, 4, 2, 1000),
-                                       (40, 8, 8, 17)])
+                                       (40, 8, 8, 17), (5, 2, 8, 128), (16, 8, 4, 2049), (3, 4, 2, 5000)])
 def test_one_split_writes_the_combined_result(gpu, b, hkv, g, n, dtype):
     """A call of one split (at most 64 tokens, or enough sequences) writes its output from the partial kernel: the
     bits of the partial pass and the combine, into strided outputs, for plain, ragged and appending calls."""
@@ -413,8 +413,11 @@ def test_one_split_writes_the_combined_result(gpu, b, hkv, g, n, dtype):
     want = out.clone()
     wide.zero_()
     plan.run()
-    # The four-wave and the two-wave work-group sum in different orders.
-    assert torch.equal(out, want) or (n <= 2048 and torch.allclose(out.float(), want.float(), rtol=2 ** -7, atol=1e-3))
+    # In between, the call's four waves and the partial pass's two sum in different orders.
+    if n <= 128 or n > 2048:
+        assert torch.equal(out, want)
+    else:
+        assert torch.allclose(out.float(), want.float(), rtol=2 ** -7, atol=1e-3)
     assert not wide[..., :32].any() and not wide[..., 160:].any()
     lens = torch.randint(0, n + 1, (b,), generator=gen, device=gpu).to(torch.int32)
     got = flash_decode.decode_attention_batched(q, k, v, SCALE, lens=lens, split=plan.split_tokens)

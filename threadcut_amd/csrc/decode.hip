@@ -606,12 +606,16 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PAGED ? 
     }
     // L >= 1 whenever a token was seen (the maximum contributes exp2(0)).
     const float inv = L == 0.f ? 0.f : __builtin_amdgcn_rcpf(L);
+    float2 y = make_float2(O0 * inv, O1 * inv);
     if constexpr (DIRECT) {
+      // Rounded to fp32 and then to the element type, as the combine reads and
+      // writes it (the compiler would take both steps in one v_fma_mix).
+      __asm__("" : "+v"(y.x), "+v"(y.y));
       uint16_t* dst = a.out + b * a.so_b + h * a.so_h + hh * a.so_g + d;
-      *reinterpret_cast<uint32_t*>(dst) = E::bits(O0 * inv) | (E::bits(O1 * inv) << 16);
+      *reinterpret_cast<uint32_t*>(dst) = E::bits(y.x) | (E::bits(y.y) << 16);
       continue;
     }
-    *reinterpret_cast<float2*>(o_out + hh * kHeadDim + d) = make_float2(O0 * inv, O1 * inv);
+    *reinterpret_cast<float2*>(o_out + hh * kHeadDim + d) = y;
     if (d == 0) l_out[hh] = (L == 0.f) ? neg_inf() : (Mx + __builtin_amdgcn_logf(L)) * kLn2;
   }
 #if TC_DECODE_STAMPS
