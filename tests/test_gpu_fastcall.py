@@ -26,6 +26,25 @@ def same(a, b):
     return a == b
 
 
+def watch(monkeypatch):
+    """Watches the native functions from here on; calling the result tells of each that was called whether it took
+    its last call."""
+    _lib.load()
+    taken, fast = {}, _lib.FAST
+
+    class Watched:
+        def __getattr__(self, name):
+            def call(*args):
+                r = getattr(fast, name)(*args)
+                taken[name] = r is not None and r is not False
+                return r
+
+            return call
+
+    monkeypatch.setattr(_lib, "FAST", Watched())
+    return lambda: taken
+
+
 def test_host_tensors_are_left_to_python():
     _lib.load()
     f, x = _lib.FAST, torch.zeros(1, 1, 1, 128, dtype=torch.float16)
@@ -65,7 +84,11 @@ def test_decode(gpu, monkeypatch, qf, cf, b, hq, hkv, n, dtype):
         pytest.skip("one head")
     q, (k, v) = query(qf, b, hq, dtype, gpu), cache(cf, b, hkv, n, dtype, gpu)
     f = lambda: attention.attention(None, q, k, v, None, scaling=0.1)[0]
-    assert same(outcome(f), general(monkeypatch, f))
+    taken = watch(monkeypatch)
+    got, heads = outcome(f), k.shape[1]
+    assert taken() == {"decode": qf in QUERIES[:3] and cf in (*CACHES[:4], "too few heads") and hq % heads == 0
+                       and hq // heads <= 8}
+    assert same(got, general(monkeypatch, f))
 
 
 @pytest.mark.gpu
@@ -88,7 +111,10 @@ def test_append(gpu, monkeypatch, new, pos, b, hq, hkv, n):
         assert layer.pending is None
         return torch.cat((out.flatten(), layer.kbuf[:, :, :n + 1].flatten(), layer.vbuf[:, :, :n + 1].flatten()))
 
-    assert same(outcome(step), general(monkeypatch, step))
+    taken = watch(monkeypatch)
+    got = outcome(step)
+    assert taken()["decode_append"] == (new in ("tokens first", "heads first"))
+    assert same(got, general(monkeypatch, step))
 
 
 @pytest.mark.gpu
@@ -111,21 +137,58 @@ def test_paged_append(gpu, monkeypatch, form, b):
         assert out is None or got is out or got.data_ptr() == out.data_ptr()
         return torch.cat((got.flatten(), c.k_pools[1].flatten(), c.v_pools[1].flatten()))
 
-    assert same(outcome(step), general(monkeypatch, step))
+    taken = watch(monkeypatch)
+    got = outcome(step)
+    assert taken().get("paged_append", False) == (form in ("plain", "out"))
+    assert same(got, general(monkeypatch, step))
+
+
+SPIN = 100_000_000  # cycles of torch.cuda._sleep's counter: tens of milliseconds or more
 
 
 @pytest.mark.gpu
-def test_native_calls_follow_the_current_stream(gpu):
-    """A call inside a stream's context is enqueued there: it waits for the work before it."""
-    q = query("tokens first", 1, 32, torch.float16, gpu)
-    k, v = cache("whole", 1, 8, 300, torch.float16, gpu)
-    want = attention.attention(None, q, k, v, None)[0]
-    k2, s = torch.zeros_like(k), torch.cuda.Stream()
-    s.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(s):
-        for _ in range(20):
-            k2.zero_()
-        k2.copy_(k)
-        got = attention.attention(None, q, k2, v, None)[0]
-    s.synchronize()
-    assert torch.equal(got, want)
+@pytest.mark.parametrize("entry", ["decode", "decode_append", "paged_append", "append_rows"])
+def test_native_calls_follow_the_current_stream(gpu, monkeypatch, entry):
+    """A call inside a stream's context is enqueued there: behind a spin and the copies that fill its input, it finds
+    the input filled."""
+    b, hkv, n = 2, 8, 300
+    src = query("tokens first", b, hkv if entry != "decode" else 32, torch.float16, gpu)
+    k, v = cache("whole", b, hkv, n, torch.float16, gpu)
+    q = query("heads first", b, 32, torch.float16, gpu)
+    if entry == "append_rows":
+        src = cache("tokens first", b, hkv, 70, torch.float16, gpu)[0]
+
+    def prepared():
+        """The call's input, empty, and the call."""
+        x = torch.zeros_like(src)
+        if entry == "decode":
+            return x, lambda: attention.attention(None, x, k, v, None)[0]
+        if entry == "paged_append":
+            c = paged.PagedKV(1, hkv, 60, 16, batch=b, device=gpu)
+            for i in range(b):
+                c.append(i, [k[i]], [v[i]])
+            c.reserve_step()
+            return x, lambda: (c.decode_append(0, q.view(b, hkv, 4, 128), x, x, 0.1), c.k_pools[0])
+        layer = kv.GrowingLayer()
+        layer.update(k, v)
+        if entry == "append_rows":
+            return x, lambda: layer.update(x, x)
+        layer.fused_append = True
+        return x, lambda: (attention.attention(None, q, *layer.update(x, x), None)[0], layer.keys)
+
+    x, call = prepared()
+    x.copy_(src)
+    want = [t.clone() for t in torch.utils._pytree.tree_leaves(call())]
+    x, call = prepared()
+    taken = watch(monkeypatch)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(SPIN)
+        x.copy_(src)
+        got = torch.utils._pytree.tree_leaves(call())
+    assert not side.query(), "the spin ended before the call was enqueued"
+    side.synchronize()
+    assert taken() == {entry: True}
+    assert len(got) == len(want) and all(torch.equal(a, w) for a, w in zip(got, want))

@@ -1,6 +1,8 @@
 """The cache appends as kernels (tc_append_rows, tc_paged_append_rows) against torch's own copies: every view a
 caller may hand over lands in the same rows bit for bit, and nothing else of the buffer changes. Views that the
 kernels do not take (misaligned, another type, a broadcast batch) go through torch and give the same."""
+import types
+
 import pytest
 import torch
 
@@ -51,7 +53,12 @@ def test_growing_layer_append(gpu, form, b, h, n, dtype):
     want_k[:, :, 7:7 + n] = k
     want_v[:, :, 7:7 + n] = v
     assert kv.rows_ok(k, layer.kbuf, n) == (form in KERNEL or form == "broadcast batch")
-    layer.update(k, v)
+    native = _lib.FAST.append_rows
+    taken = []
+    with pytest.MonkeyPatch.context() as m:
+        m.setattr(_lib, "FAST", types.SimpleNamespace(append_rows=lambda *a: taken.append(native(*a)) or taken[-1]))
+        layer.update(k, v)
+    assert taken == [form in KERNEL or form == "broadcast batch" and b == 1]
     assert layer.n == 7 + n
     assert torch.equal(layer.kbuf, want_k) and torch.equal(layer.vbuf, want_v)
 
@@ -63,6 +70,13 @@ def test_append_under_autograd_stays_with_torch(gpu):
     layer.update(k, k)
     layer.keys.float().sum().backward()
     assert torch.equal(k.grad, torch.ones_like(k))
+
+
+def watch_rows(monkeypatch):
+    """What every later PagedKV._write_rows call returns: True where the kernel took the rows."""
+    taken, write = [], paged.PagedKV._write_rows
+    monkeypatch.setattr(paged.PagedKV, "_write_rows", lambda *a: taken.append(write(*a)) or taken[-1])
+    return taken
 
 
 class Config:
@@ -198,16 +212,18 @@ def test_append_of_more_rows_than_the_kernel_takes(gpu, monkeypatch, native):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("form", [f for f in KERNEL + TORCH if f != "broadcast batch"])
 @pytest.mark.parametrize("layers,P,n", [(1, 16, 1), (3, 64, 65), (70, 16, 37)])
-def test_paged_append(gpu, form, layers, P, n, dtype):
+def test_paged_append(gpu, monkeypatch, form, layers, P, n, dtype):
     """PagedKV.append (every layer in one launch; 70 layers take two) from a page that is partly full."""
     h = 3
     cache = paged.PagedKV(layers, h, 12, P, dtype=dtype, device=gpu)
     cache.table.free.reverse()
     start = [rows("heads first", 1, h, 5, dtype, gpu, i) for i in range(layers)]
     cache.append(0, start, start)
+    taken = watch_rows(monkeypatch)
     ks = [rows(form, 1, h, n, dtype, gpu, 100 + i) for i in range(layers)]
     vs = [rows("tokens first", 1, h, n, dtype, gpu, 300 + i)[0] for i in range(layers)]
     cache.append(0, ks, vs)
+    assert taken == [form in KERNEL]
     for i in range(layers):
         k, v = cache.gather(i)
         assert torch.equal(k, torch.cat((start[i], ks[i].to(dtype)), 2)[0])
@@ -221,15 +237,17 @@ def test_paged_append(gpu, form, layers, P, n, dtype):
 
 @pytest.mark.parametrize("form", KERNEL + ["misaligned", "float32"])
 @pytest.mark.parametrize("b,n", [(1, 40), (3, 17)])
-def test_paged_layer_update(gpu, form, b, n):
+def test_paged_layer_update(gpu, monkeypatch, form, b, n):
     """A paged cache layer's update writes every sequence's rows with one launch."""
     cache = paged.new_paged_cache(Config(), 40, 16, batch=b)
     first = rows("heads first", b, 4, 9, torch.float16, gpu, 5)
     k, v = rows(form, b, 4, n, torch.float16, gpu, 6), rows("tokens first", b, 4, n, torch.float16, gpu, 7)
     for i in range(2):
         cache.update(first, first, i)
+    taken = watch_rows(monkeypatch)
     for i in range(2):
         cache.update(k, v, i)
+    assert taken == [form in KERNEL] * 2
     store = paged.state_of(cache).kv
     for i in range(2):
         for j in range(b):
