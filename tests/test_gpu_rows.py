@@ -169,6 +169,7 @@ def test_append_outside_inference_mode_keeps_its_refusal(gpu, monkeypatch, kind)
         s.append(rows("heads first", 1, 2, 5, torch.float16, gpu, 2), rows("heads first", 1, 2, 5, torch.float16, gpu, 2))
 
 
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
 @pytest.mark.parametrize("kind", STORES)
 def test_append_is_recorded_by_tracing(gpu, monkeypatch, kind):
     """torch.jit.trace, make_fx and torch.compile record the write: what they return follows new inputs."""

@@ -54,8 +54,9 @@ constexpr int kRowBytes = 2 * kHeadDim;  // a K or V row in LDS (unpadded)
 // (key <= n - q_len + token), so its elements are tested arithmetically.
 enum : int { TILE_SKIP = 0, TILE_FULL = 1, TILE_MIXED = 2, TILE_CAUSAL = 3 };
 
-// Waves per SIMD the register allocation targets: 2 leaves 256 registers a
-// lane and matches the two 68 KB work-groups the LDS of a CU holds.
+// Waves per SIMD the register allocation targets: 2 leaves 256 registers a lane
+// and matches what the 160 KB LDS of a CU holds, two work-groups of four waves
+// (64 KB of tile buffers each) or one of eight (128 KB).
 #ifndef TC_PREFILL_WAVES
 #define TC_PREFILL_WAVES 2
 #endif
@@ -99,7 +100,8 @@ struct PrefillArgs {
   int64_t tok_pitch;
   int64_t pool_bytes_k, pool_bytes_v;
 #if TC_PREFILL_STAMPS
-  // Per wave (work-group * 4 + wave), kStampWords words: a header of 8 (shader
+  // The shapes of one key group only (Wide). Per wave (work-group * 4 + wave),
+  // kStampWords words: a header of 8 (shader
   // clock and realtime clock at the start, the same at the end, HW_REG_HW_ID
   // | HW_REG_XCC_ID << 32, tiles recorded), then 5 shader-clock stamps per
   // tile (its start, QK^T issued, softmax done, P.V issued, its loads landed).

@@ -37,7 +37,7 @@ struct RowArgs {
   int64_t d_b, d_h, d_t;            // destination strides (paged: page, head, slot)
   const int64_t* slots;             // paged: [batch, rows, 2] of (page, slot); null: contiguous
   int64_t rows;
-  int layers, heads;
+  int layers;
   int pages, page_tokens;
 };
 
@@ -156,7 +156,6 @@ int write_rows(const void* const* ks, const int64_t* k_st, const void* const* vs
     a.slots = d.slots;
     a.rows = rows;
     a.layers = nl;
-    a.heads = heads;
     a.pages = d.pages;
     a.page_tokens = d.page_tokens;
     launch(a, dim3(heads, static_cast<unsigned>(tiles), static_cast<unsigned>(batch * 2 * nl)), s);
