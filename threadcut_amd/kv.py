@@ -124,7 +124,7 @@ def rows_ok(t, buf, rows):
 def _append_rows(kbuf, vbuf, row0, k, v):
     """Rows of the new tokens k/v to rows row0 .. of both buffers: one launch (tc_append_rows) for K and V where
     the kernel takes them, torch's two copies otherwise (host tensors, other types, head dims or broadcasts)."""
-    fast = None if torch.compiler.is_compiling() else _lib.FAST
+    fast = None if torch.compiler.is_dynamo_compiling() else _lib.FAST  # (which asks for other tracing itself)
     if fast is not None and kbuf.is_cuda and fast.append_rows(kbuf, vbuf, row0, k, v,
                                                               _lib.raw_stream(kbuf.get_device())):
         return
