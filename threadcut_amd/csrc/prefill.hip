@@ -1130,10 +1130,10 @@ struct Plan {
 // - A chunk on a longer cache is split to fill the CUs once (a second round
 //   would double the call), into at most 32 splits of at least 256 keys.
 //   - T <= 5: Narrow, Wide where W64 > C. A Deep tile of 128 keys is mostly empty
-//     there: 14 tokens on 43 of 32 heads 6.5 us against 7.8 Deep, 6.3 Wide; at T = 2
-//     0.83 of Deep's time over 366 shapes, 0.97 at 5, 1.02 at 6 and 7.
+//     there: 14 tokens on 43 of 32 heads 6.5 us against 7.8 Deep, 6.3 Wide; 0.92 of
+//     Deep's time at T = 2 (366 shapes), 0.97 at 5, 1.02 at 6 and 7.
 //   - Deep for few rows (W64 <= C / 6) or short caches (n <= 4096 and two splits, W64
-//     <= C / 2; n <= 3072, W64 <= 7/8 C: 0.82 of Wide's time with T in [16, 24), 1.03
+//     <= C / 2; n <= 3072, W64 <= 7/8 C: 0.78 of Wide's time with T in [16, 24), 1.03
 //     in [56, 64)):
 //     3 tokens on 9000: 15.6 against 17.3 Wide, 16.9 Tall; 150 on 1500: 19.7,
 //     22.3, 22.2; 400 on 3000: 38.1, 43.0, 41.7.
