@@ -225,3 +225,14 @@ def test_library_chosen_splits_need_the_workspace_the_query_tells(gpu, hq, hkv, 
             else:
                 assert rc == _lib.TC_OK, lib.tc_last_error()
                 check(out, want, torch.float16)
+
+
+def test_masks_made_in_inference_mode(gpu):
+    """Such a mask has no version counter: each call classifies it as it is then."""
+    hq, hkv, ql, n = 32, 8, 100, 900
+    q, k, v = workloads.prefill_inputs(4, q_len=ql, n=n, q_heads=hq, kv_heads=hkv, device=gpu)
+    with torch.inference_mode():
+        m, vis = masks("chunk", ql, n, 1, gpu, 0)
+        check(prefill.prefill_attention(q, k, v, m, SCALE), reference(q, k, v, vis, SCALE), torch.float16)
+        m[..., 100:500] = False
+        check(prefill.prefill_attention(q, k, v, m, SCALE), reference(q, k, v, m[:, 0], SCALE), torch.float16)

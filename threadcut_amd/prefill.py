@@ -130,14 +130,15 @@ def prefill_attention(query, key, value, attention_mask=None, scale=None, is_cau
 # pass and hands the same tensor to every layer, so the map is built once per
 # pass; it is rebuilt when the mask object, its version or the geometry change.
 # A captured call builds its own: a replay must not read a map that it did not
-# make, of the mask as it was before.
+# make, of the mask as it was before. So does a call on a mask made in inference
+# mode: such a tensor has no version to tell of a change.
 _tile_cache = None
 
 
 def mask_tiles(mask, q_heads, kv_heads):
     """uint8 tile map of a bool mask [b|1, 1, q, n] (``tc_prefill_mask_tiles``), cached per mask."""
     global _tile_cache
-    if torch.cuda.is_current_stream_capturing():
+    if mask.is_inference() or torch.cuda.is_current_stream_capturing():
         return _build_tiles(mask, q_heads, kv_heads)
     key = (mask._version, mask.shape, mask.stride(), mask.data_ptr(), q_heads, kv_heads)
     c = _tile_cache
