@@ -4,6 +4,7 @@ import ctypes
 import importlib.util
 import os
 import re
+import struct
 import sys
 import types
 
@@ -217,6 +218,16 @@ def test_append_validation(lib):
     assert paged(pages=0) == _lib.TC_ERR_INVALID_ARGUMENT
     assert paged(k=_lib.ptr_array([0])) == _lib.TC_ERR_INVALID_ARGUMENT
     assert paged(layers=0, slots=None) == _lib.TC_OK
+
+
+def test_native_paths_hold_no_thread_local_of_their_own():
+    """Loading a module with a thread-local segment that nothing touches leaves every thread-local access of the
+    process (torch has many, the HIP runtime too) on the loader's slow path."""
+    elf = open(os.path.join(os.path.dirname(_lib.LIB_PATH), "_fast.so"), "rb").read()
+    offset, = struct.unpack_from("<Q", elf, 32)
+    size, count = struct.unpack_from("<HH", elf, 54)
+    types_ = {struct.unpack_from("<I", elf, offset + i * size)[0] for i in range(count)}
+    assert 1 in types_ and 7 not in types_  # PT_LOAD, PT_TLS
 
 
 @pytest.mark.parametrize("fault", ["absent", "another torch"])

@@ -79,7 +79,9 @@ def _compile_fast(obj):
     from torch.utils.cpp_extension import include_paths
 
     system = [x for p in (*include_paths(), sysconfig.get_paths()["include"]) for x in ("-isystem", p)]
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+    # NDEBUG: without it pybind11's headers add a thread-local counter, and a module with a thread-local segment that
+    # nothing touches slows down every thread-local access of the process (an empty tensor 0.98 -> 1.24 us).
+    cmd = ["g++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f'-DTC_TORCH_VERSION="{torch.__version__}"', *system, "-c", os.path.join(CSRC, "host", "fastcall.cpp"), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
