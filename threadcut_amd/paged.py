@@ -394,8 +394,9 @@ class PagedKV:
             mptr, mst = m.data_ptr(), pf._mask_strides(m)
         lib = _lib.load()
         kp, vp = self.k_pools[layer], self.v_pools[layer]
-        splits, nbytes = pf._plan(self.device.index, b, ql, n, hq, self.kv_heads, None)
-        with _on_device(self.device):
+        with torch.cuda.device(self.device):
+            splits = pf.num_splits(b, ql, n, hq, self.kv_heads)
+            nbytes = lib.tc_prefill_workspace_bytes(b, ql, hq, splits)
             ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=self.device)
             rc = lib.tc_prefill_paged_attention(
                 query.data_ptr(), pf._strides(query, (0, 1, 2)), kp.data_ptr(), vp.data_ptr(), self._strides(),

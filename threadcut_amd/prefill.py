@@ -9,13 +9,11 @@ K and V in LDS once for all of them and runs QKᵀ and PV on the matrix cores wi
 online softmax. This module checks tensors and passes pointers, strides and
 the current stream.
 """
-import functools
 import weakref
 
 import torch
 
 from . import _lib
-from .flash_decode import _on_device
 
 HEAD_DIM = 128
 GROUPS = (1, 2, 4, 8)
@@ -58,14 +56,6 @@ def num_splits(batch, q_len, n_tokens, q_heads, kv_heads):
     if s < 0:
         _lib.check(-s, "tc_prefill_num_splits")
     return s
-
-
-@functools.lru_cache(maxsize=1024)
-def _plan(device_index, b, q, n, hq, hkv, splits):
-    """(splits, workspace bytes) of a call; the library plans for the current device (its CU count)."""
-    with torch.cuda.device(device_index):
-        s = int(splits) if splits else num_splits(b, q, n, hq, hkv)
-    return s, _lib.load().tc_prefill_workspace_bytes(b, q, hq, s)
 
 
 def prefill_attention(query, key, value, attention_mask=None, scale=None, is_causal=False, out=None, splits=None):
@@ -112,8 +102,10 @@ def prefill_attention(query, key, value, attention_mask=None, scale=None, is_cau
         mask_ptr, mask_strides = m.data_ptr(), _mask_strides(m)
     scale = scale if scale is not None else d ** -0.5
     lib = _lib.load()
-    s, ws_bytes = _plan(query.get_device(), b, q, n, hq, hkv, splits)
-    with _on_device(query.device):
+    # The library plans splits for the current device (its CU count).
+    with torch.cuda.device(query.device):
+        s = int(splits) if splits else num_splits(b, q, n, hq, hkv)
+        ws_bytes = lib.tc_prefill_workspace_bytes(b, q, hq, s)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device) if ws_bytes else None
         rc = lib.tc_prefill_attention(
             query.data_ptr(), _strides(query, (0, 1, 2)), key.data_ptr(), _strides(key, (0, 1, 2), 2),
@@ -159,7 +151,7 @@ def _build_tiles(mask, q_heads, kv_heads):
     nbytes = lib.tc_prefill_tiles_bytes(q, n, mb, q_heads, kv_heads)
     tiles = torch.empty(max(1, nbytes), dtype=torch.uint8, device=mask.device)
     st = _mask_strides(m, batch=mb > 1)
-    with _on_device(mask.device):
+    with torch.cuda.device(mask.device):
         rc = lib.tc_prefill_mask_tiles(m.data_ptr(), st, mb, q, n, q_heads, kv_heads, tiles.data_ptr(),
                                        tiles.numel(), _lib.stream_of(mask.device))
     _lib.check(rc, "tc_prefill_mask_tiles")
